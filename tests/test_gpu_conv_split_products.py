@@ -101,3 +101,57 @@ def test_operands_without_finite_parts(be, orc, shape, what):
         fine = np.isfinite(e)
         mag = np.abs(e[fine & (np.abs(e) < 1e20)]).max() if (fine & (np.abs(e) < 1e20)).any() else 1.0
         np.testing.assert_allclose(g[fine], e[fine], rtol=RTOL, atol=ATOL * max(1.0, float(mag)), err_msg=op)
+
+
+def products64(x, k, dy, s):
+    """The three products in float64, one filter tap at a time."""
+    x, k, dy = (a.astype(np.float64) for a in (x, k, dy))
+    N, H, W, C = x.shape
+    kh, kw, _, O = k.shape
+    Ho, Wo = dy.shape[1:3]
+    pt, pl = (same_pad(n, f, s)[0] // 2 for n, f in ((H, kh), (W, kw)))
+    xp = np.zeros((N, max((Ho - 1) * s + kh, H + pt), max((Wo - 1) * s + kw, W + pl), C))
+    xp[:, pt:pt + H, pl:pl + W] = x
+    y, dxp, dk = np.zeros((N, Ho, Wo, O)), np.zeros_like(xp), np.zeros_like(k)
+    for i in range(kh):
+        for j in range(kw):
+            at = np.s_[:, i:i + (Ho - 1) * s + 1:s, j:j + (Wo - 1) * s + 1:s]
+            y += xp[at] @ k[i, j]
+            dxp[at] += dy @ k[i, j].T
+            dk[i, j] = xp[at].reshape(-1, C).T @ dy.reshape(-1, O)
+    return {"fwd": y, "dx": dxp[:, pt:pt + H, pl:pl + W], "dk": dk}
+
+
+SPARSE = [(shape, op) for shape in SHAPES[:5] for op in ("fwd", "dx", "dk")]
+
+
+@pytest.mark.parametrize("live", ["one", 0.1, 0.5, "positive"])
+@pytest.mark.parametrize("shape,op", SPARSE)
+def test_no_less_accurate_on_sparse_operands(be, shape, op, live):
+    """As above where few of a sum's products are not zero (activations and gradients behind a relu): fp32 rounds
+    such a sum once per product, and the parts of one product must not cost more.  one: one product on average;
+    positive: all of them, of one sign.  1.1: the three products of parts that are left out add 3 % to the error of a
+    single product, the rest is the scatter of two norms over thousands of elements."""
+    print("shape", shape, op, live, flush=True)
+    x, k, dy = rand_conv_inputs(17, *shape)
+    s = shape[-1]
+    rng = np.random.default_rng(18)
+    terms = {"fwd": k[..., 0].size, "dx": k[:, :, 0].size / s ** 2, "dk": dy[..., 0].size}[op]
+    if live == "positive":
+        x, k, dy = np.abs(x), np.abs(k), np.abs(dy)
+    else:
+        part = 1.0 / terms if live == "one" else live
+        if op == "dx":
+            dy = np.where(rng.random(dy.shape) < part, dy, np.float32(0))
+        else:
+            x = np.where(rng.random(x.shape) < part, x, np.float32(0))
+    got = products(be, x, k, dy, s)[op].astype(np.float64)
+    be.lib.dh_debug_force_generic_conv(1)
+    try:
+        plain = products(be, x, k, dy, s)[op].astype(np.float64)
+    finally:
+        be.lib.dh_debug_force_generic_conv(0)
+    exact = products64(x, k, dy, s)[op]
+    err, yard, norm = np.linalg.norm(got - exact), np.linalg.norm(plain - exact), np.linalg.norm(exact)
+    print("  relative error %.3g, fp32 products %.3g: %.2f" % (err / norm, yard / norm, err / yard), flush=True)
+    assert err <= 1.1 * yard
