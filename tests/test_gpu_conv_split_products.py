@@ -123,7 +123,7 @@ def products64(x, k, dy, s):
 
 
 SPARSE = [(shape, op) for shape in SHAPES[:5] for op in ("fwd", "dx", "dk")]
-SPARSE += [(shape, "fwd") for shape in SHAPES[5:]]
+SPARSE += [(shape, op) for shape in SHAPES[5:] for op in ("fwd", "dx")]
 
 
 @pytest.mark.parametrize("live", ["one", 0.1, 0.5, "positive"])
