@@ -155,3 +155,38 @@ def test_no_less_accurate_on_sparse_operands(be, shape, op, live):
     err, yard, norm = np.linalg.norm(got - exact), np.linalg.norm(plain - exact), np.linalg.norm(exact)
     print("  relative error %.3g, fp32 products %.3g: %.2f" % (err / norm, yard / norm, err / yard), flush=True)
     assert err <= 1.1 * yard
+
+
+@pytest.mark.parametrize("what", ["small times large", "subnormal times large", "small beside ordinary"])
+@pytest.mark.parametrize("shape", SHAPES)
+def test_small_operands(be, shape, what):
+    """Operands whose parts bf16 holds only in part (below 2^-109) or not at all, where their products count: beside
+    a large partner, or as the one small image (filter gradient: the one small channel) of a tile of ordinary ones.
+    The slice of the result that they make is as close to float64 sums as the fp32 kernel's (1.1: as above)."""
+    print("shape", shape, what, flush=True)
+    s = shape[-1]
+    x, k, dy = rand_conv_inputs(19, *shape)
+    inputs = {"fwd": (x, k, dy), "dx": (x, k, dy), "dk": (x, k, dy)}
+    where = {"fwd": np.s_[:], "dx": np.s_[:], "dk": np.s_[:]}
+    if what == "small beside ordinary":
+        x0, dy0, xc = x.copy(), dy.copy(), x.copy()
+        x0[0] *= np.float32(1e-36)
+        dy0[0] *= np.float32(1e-36)
+        xc[..., 0] *= np.float32(1e-36)
+        inputs = {"fwd": (x0, k, dy), "dx": (x, k, dy0), "dk": (xc, k, dy)}
+        where = {"fwd": np.s_[0], "dx": np.s_[0], "dk": np.s_[:, :, 0]}
+    else:
+        small, large = (np.float32(v) for v in ((1e-37, 1e16) if what == "small times large" else (1e-41, 1e20)))
+        inputs = {"fwd": (x * small, k * large, dy), "dx": (x, k * large, dy * small), "dk": (x * small, k, dy * large)}
+    for op in inputs:
+        got = products(be, *inputs[op], s)[op]
+        be.lib.dh_debug_force_generic_conv(1)
+        try:
+            plain = products(be, *inputs[op], s)[op]
+        finally:
+            be.lib.dh_debug_force_generic_conv(0)
+        exact = products64(*inputs[op], s)[op][where[op]]
+        err, yard = (np.linalg.norm(r[where[op]].astype(np.float64) - exact) for r in (got, plain))
+        norm = np.linalg.norm(exact)
+        print("  %s: relative error %.3g, fp32 products %.3g" % (op, err / norm, yard / norm), flush=True)
+        assert err <= 1.1 * yard, op
