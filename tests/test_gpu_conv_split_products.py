@@ -190,3 +190,26 @@ def test_small_operands(be, shape, what):
         norm = np.linalg.norm(exact)
         print("  %s: relative error %.3g, fp32 products %.3g" % (op, err / norm, yard / norm), flush=True)
         assert err <= 1.1 * yard, op
+
+
+@pytest.mark.parametrize("op", ["fwd", "dx"])
+def test_tile_width_changes_no_result_beside_infinities(be, op):
+    """The two tile widths that a launch may be measured with give the same bits where an infinity makes part of a
+    tile form its products again in fp32: one filter column of the 160, whose neighbours stay finite."""
+    shape = (16, 16, 16, 64, 5, 5, 160, 2) if op == "fwd" else (16, 16, 16, 160, 5, 5, 64, 2)
+    x, k, dy = rand_conv_inputs(23, *shape)
+    if op == "fwd":
+        k[2, 2, 3, 5] = np.inf
+    else:
+        k[2, 2, 5, 3] = np.inf
+    got = []
+    be.lib.dh_debug_force_splitk(1)
+    try:
+        for width in (64, 128):
+            be.lib.dh_debug_force_tile_width(width)
+            got.append(be.conv2d(x, k, (2, 2)) if op == "fwd" else be.conv2d_input_grad(dy, k, 2, x.shape[1:3]))
+    finally:
+        be.lib.dh_debug_force_tile_width(0)
+        be.lib.dh_debug_force_splitk(0)
+    assert np.isfinite(got[0][..., 6:]).all() and not np.isfinite(got[0][..., 5]).all()
+    np.testing.assert_array_equal(got[0], got[1])
