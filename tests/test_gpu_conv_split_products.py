@@ -213,3 +213,47 @@ def test_tile_width_changes_no_result_beside_infinities(be, op):
         be.lib.dh_debug_force_splitk(0)
     assert np.isfinite(got[0][..., 6:]).all() and not np.isfinite(got[0][..., 5]).all()
     np.testing.assert_array_equal(got[0], got[1])
+
+
+# the pixel order of tiles that span two pixels (batch half the tile height: 128 rows 128 or 64 wide, 64 rows), a batch
+# that is no multiple of 16, and the image layer
+PAIRS = [(64, 8, 8, 144, 5, 5, 160, 2), (64, 8, 8, 32, 5, 5, 64, 2), (32, 2, 4, 16, 2, 2, 48, 2), (5, 9, 7, 32, 3, 3, 48, 1),
+         (3, 64, 64, 3, 5, 5, 64, 2)]
+
+
+@pytest.mark.parametrize("odd", [np.inf, np.nan, 1e30])
+@pytest.mark.parametrize("where", ["first", "second", "filter"])
+@pytest.mark.parametrize("shape", PAIRS)
+def test_operands_without_finite_parts_in_paired_launches(be, orc, shape, where, odd):
+    """Operands whose products are formed again in fp32 (infinity, NaN, a sum beyond 2^80) in either instance of a
+    paired launch or in the filter, and in the single launches: the results are the oracle's, non-finite ones where
+    it has them.  The odd values sit where every tap they meet is inside the image."""
+    print("shape", shape, where, odd, flush=True)
+    N, H, W, C, kh, kw, O, s = shape
+    (x1, k, dy1), (x2, _, dy2) = (rand_conv_inputs(seed, *shape) for seed in (29, 31))
+    k[np.abs(k) < 1e-4] = 1e-4
+    i, j = dy1.shape[1] // 2, dy1.shape[2] // 2
+    if where == "filter":
+        k[kh // 2, kw // 2, C - 1, O - 3] = odd
+    else:
+        (x1 if where == "first" else x2)[N // 2, H // 2, W // 2, C - 1] = odd
+        (dy1 if where == "first" else dy2)[N - 1, i, j, 1] = odd
+    pads = (same_pad(H, kh, s)[0], same_pad(W, kw, s)[0])
+    orc.set_threads(8)
+    with np.errstate(all="ignore"):
+        exp1, exp2 = products(orc, x1, k, dy1, s), products(orc, x2, k, dy2, s)
+        both = exp1["dk"] + exp2["dk"]
+    got = {"fwd 1": (be.conv2d(x1, k, (s, s)), exp1["fwd"]), "dx 2": (be.conv2d_input_grad(dy2, k, s, (H, W)), exp2["dx"]),
+           "dk 2": (be.conv2d_kernel_grad(dy2, x2, s, pads), exp2["dk"])}
+    y1, y2 = be.conv2d_pair(x1, x2, k, (s, s))
+    got.update({"pair fwd 1": (y1, exp1["fwd"]), "pair fwd 2": (y2, exp2["fwd"])})
+    if C % 16 == 0:
+        g1, g2 = be.conv2d_input_grad_pair(dy1, dy2, k, s, (H, W))
+        got.update({"pair dx 1": (g1, exp1["dx"]), "pair dx 2": (g2, exp2["dx"])})
+    got["pair dk"] = (be.conv2d_kernel_grad_pair(dy1, x1, dy2, x2, s, pads), both)
+    for op, (g, e) in got.items():
+        for kind in (np.isnan, np.isposinf, np.isneginf):
+            np.testing.assert_array_equal(kind(g), kind(e), err_msg=op)
+        fine = np.isfinite(e)
+        plain = np.abs(e[fine & (np.abs(e) < 1e20)])
+        np.testing.assert_allclose(g[fine], e[fine], rtol=RTOL, atol=ATOL * max(1.0, float(plain.max(initial=0))), err_msg=op)
