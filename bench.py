@@ -39,8 +39,8 @@ ROOT = os.path.dirname(os.path.abspath(__file__))
 sys.path.insert(0, ROOT)
 import __graft_entry__ as ge  # noqa: E402
 
-# MI355X dense fp32 matrix peak.  The convolution kernels form fp32 products from six bf16 ones (2500 / 6 = 417 TFLOP/s by
-# the bf16 peak), so their fractions of this peak may exceed 1.
+# MI355X dense fp32 matrix peak.  The convolution kernels (but for the general one and the image layer's filter gradient) form
+# fp32 products from six bf16 ones (2500 / 6 = 417 TFLOP/s by the bf16 peak), so their fractions of this peak may exceed 1.
 PEAK_FP32_MFMA_TFLOPS = 157.3
 PEAK_HBM_GBS = 8000.0
 CALIBRATION_COPY_BYTES = 256 << 20

@@ -389,7 +389,8 @@ __device__ __forceinline__ float sum_of_parts(const float* __restrict__ g, unsig
     return s;
 }
 
-// One wavefront per column.  Bound by the latency of the loads, which one launch has 64 columns at most to hide.
+// One wavefront per column.  Bound by the latency of the loads: the few hundred columns of a layer (64 of the
+// widest) are a wavefront or two per compute unit, with nothing else to hide it.
 __global__ __launch_bounds__(TPB) void colsum_stage2(const float* __restrict__ partial, float* __restrict__ out,
                                                      uint32_t cols, uint32_t chunks)
 {

@@ -1,7 +1,8 @@
-"""The convolution kernels form fp32 products from bf16 parts (csrc/conv_igemm.inc, csrc/conv_small.hip).  Two properties
-of that: it is no less accurate than the general kernel, which multiplies in fp32 (each against float64 sums),
-and operands whose parts are not finite -- infinities, NaNs, magnitudes next to the largest float -- give what
-plain fp32 arithmetic gives."""
+"""The convolution kernels form fp32 products from bf16 parts (csrc/conv_igemm.inc, csrc/conv_small.hip; the image layer's
+filter gradient multiplies in fp32).  Two properties of that: it is no less accurate than the general kernel, which
+multiplies in fp32 (each against float64 sums; dense, sparse and small operands, sums of one sign), and operands whose
+parts are not finite -- infinities, NaNs, magnitudes next to the largest float -- give what plain fp32 arithmetic
+gives, in single and paired launches and with either tile width."""
 import numpy as np
 import pytest
 
@@ -31,11 +32,11 @@ def be():
     return ge.load_package().HipBackend(0)
 
 
-def products(be, x, k, dy, s, dy_dk=None):
+def products(be, x, k, dy, s):
     H, W = x.shape[1:3]
     pads = (same_pad(H, k.shape[0], s)[0], same_pad(W, k.shape[1], s)[0])
     return {"fwd": be.conv2d(x, k, (s, s)), "dx": be.conv2d_input_grad(dy, k, s, (H, W)),
-            "dk": be.conv2d_kernel_grad(dy if dy_dk is None else dy_dk, x, s, pads)}
+            "dk": be.conv2d_kernel_grad(dy, x, s, pads)}
 
 
 @pytest.mark.parametrize("scale", ["one", "wide", "tiny"])
@@ -44,24 +45,22 @@ def test_no_less_accurate_than_fp32_products(be, orc64, shape, scale):
     """Error against float64 sums, in the 2-norm over a result of thousands of elements: at most 1.1 times that of
     the fp32 kernel (equal in expectation or better; the ratio of two such norms scatters by a few percent).
     wide: magnitudes over 20 binades, so that the low parts of large values meet the high parts of small ones.
-    tiny: activations around 1e-35, whose low parts bf16 only holds as subnormals."""
+    tiny: activations around 1e-35, whose low parts bf16 holds as subnormals only, unless they are scaled first."""
     print("shape", shape, scale, flush=True)
     x, k, dy = rand_conv_inputs(11, *shape)
-    dy_dk = dy
     if scale == "wide":
         rng = np.random.default_rng(12)
         x, dy = (a * np.exp2(rng.uniform(-10, 10, a.shape)).astype(np.float32) for a in (x, dy))
-        dy_dk = dy
     if scale == "tiny":
         x, dy = x * np.float32(1e-35), dy * np.float32(1e-35)
     s = shape[-1]
-    got = products(be, x, k, dy, s, dy_dk)
+    got = products(be, x, k, dy, s)
     be.lib.dh_debug_force_generic_conv(1)
     try:
-        plain = products(be, x, k, dy, s, dy_dk)
+        plain = products(be, x, k, dy, s)
     finally:
         be.lib.dh_debug_force_generic_conv(0)
-    exact = products(orc64, x, k, dy, s, dy_dk)
+    exact = products(orc64, x, k, dy, s)
     for op in got:
         e64 = exact[op].astype(np.float64)
         err, yard = (np.linalg.norm(r[op].astype(np.float64) - e64) for r in (got, plain))
