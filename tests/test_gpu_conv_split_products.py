@@ -256,3 +256,31 @@ def test_operands_without_finite_parts_in_paired_launches(be, orc, shape, where,
         fine = np.isfinite(e)
         plain = np.abs(e[fine & (np.abs(e) < 1e20)])
         np.testing.assert_allclose(g[fine], e[fine], rtol=RTOL, atol=ATOL * max(1.0, float(plain.max(initial=0))), err_msg=op)
+
+
+@pytest.mark.parametrize("pair", [False, True])
+@pytest.mark.parametrize("shape", [
+    (1, 3, 3, 16, 3, 3, 20, 1),       # less than one slab of 16 output pixels
+    (5, 1, 1, 48, 1, 1, 8, 1),        # an image a pixel
+    (37, 1, 2, 20, 2, 1, 144, 1),     # two, runs of eight over four images, the last slab part empty
+    (7, 2, 5, 32, 3, 3, 48, 1),       # runs that cross rows and images
+    (9, 7, 3, 12, 5, 4, 36, 2),       # a row of two pixels, most taps of a pixel in the padding
+    (17, 6, 6, 260, 2, 2, 136, 2),    # 128 x 128 tiles, rows and columns left over
+])
+def test_filter_gradient_of_any_batch(be, shape, pair):
+    """Batches that are no multiple of 16: the output pixels of a slab are decoded eight at a time and may belong to any
+    rows and images.  Element by element within the error of any fp32 summation of n products (n + 2: their own
+    rounding and the last one's)."""
+    print("shape", shape, pair, flush=True)
+    H, W, s = shape[1], shape[2], shape[-1]
+    (x, k, dy), (x2, _, dy2) = (rand_conv_inputs(seed, *shape) for seed in (37, 41))
+    pads = (same_pad(H, shape[4], s)[0], same_pad(W, shape[5], s)[0])
+    exact, mag = (products64(f(x), k, f(dy), s)["dk"] for f in (np.asarray, np.abs))
+    terms = dy[..., 0].size
+    if pair:
+        got = be.conv2d_kernel_grad_pair(dy, x, dy2, x2, s, pads)
+        exact, mag = (a + products64(f(x2), k, f(dy2), s)["dk"] for a, f in ((exact, np.asarray), (mag, np.abs)))
+        terms *= 2
+    else:
+        got = be.conv2d_kernel_grad(dy, x, s, pads)
+    assert (np.abs(got - exact) <= (terms + 2) * 2.0 ** -24 * mag).all()
