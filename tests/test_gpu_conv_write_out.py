@@ -1,0 +1,119 @@
+"""The write-out of the buffer-load convolution kernel and the sums of its slices: every activation with and without a
+bias, whole and split, with 16-byte and with single stores, and filter gradients whose many slices are shared by
+several threads."""
+import numpy as np
+import pytest
+
+from common import rand_conv_inputs, same_pad
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def A():
+    import __graft_entry__ as ge
+    A = ge.load_package().hipabi
+    A.check(A.load().dh_init(0))
+    return A
+
+
+def device(a):
+    import torch
+    return torch.from_numpy(np.ascontiguousarray(a)).cuda()
+
+
+def room(n, offset):
+    """A device tensor of n floats whose address is a multiple of 16 plus 4 * offset."""
+    import torch
+    return torch.full((n + 4,), np.nan, device="cuda")[offset:offset + n]
+
+
+@pytest.mark.parametrize("offset", [0, 1])
+@pytest.mark.parametrize("splits", [1, 3])
+@pytest.mark.parametrize("shape", [(3, 9, 7, 16, 3, 3, 36, 1), (2, 20, 20, 16, 3, 3, 132, 1)])   # one and two column tiles, remainders
+def test_activations(A, shape, splits, offset):
+    """The activation of (product + bias), element by element, from the product alone as the same launch plan gives it: exact
+    where the activation is one multiplication or none, else within 1e-6 (two roundings of tanh and exp in 32 bits)."""
+    import torch
+    print("shape", shape, "splits", splits, "offset", offset, flush=True)
+    N, H, W, C, kh, kw, O, s = shape
+    x, k, _ = rand_conv_inputs(5, *shape)
+    rng = np.random.default_rng(6)
+    bias = rng.standard_normal(O).astype(np.float32)
+    bias[:3] = -np.inf, np.nan, np.inf
+    lib, P = A.load(), torch.Tensor.data_ptr
+    (ph, Ho), (pw, Wo) = A.same_pad(H, kh, s), A.same_pad(W, kw, s)
+    xd, kd, bd = device(x), device(k), room(O, offset)
+    bd.copy_(device(bias))
+    geom = (N, H, W, C, kh, kw, O, s, s, ph // 2, pw // 2, Ho, Wo)
+
+    def run(b, act, alpha):
+        y = room(N * Ho * Wo * O, offset)
+        A.check(lib.dh_conv2d_fwd(P(xd), P(kd), P(y), *geom, b, act, alpha, None))
+        return y.cpu().numpy().reshape(-1, O)
+
+    lib.dh_debug_force_splitk(splits)
+    try:
+        plain = run(None, A.ACT_NONE, 0.0)
+        assert np.isfinite(plain).all()
+        for b in (None, bias):
+            z = plain if b is None else plain + b
+            below = z < 0
+            expected = {
+                A.ACT_NONE: z,
+                A.ACT_RELU: np.where(below, np.float32(0), z),
+                A.ACT_LEAKY: np.where(below, np.float32(0.2) * z, z),
+                A.ACT_TANH: np.tanh(z.astype(np.float64)),
+                A.ACT_SIGMOID: 1 / (1 + np.exp(-z.astype(np.float64))),
+            }
+            for act, exp in expected.items():
+                got = run(None if b is None else P(bd), act, 0.2)
+                if act in (A.ACT_TANH, A.ACT_SIGMOID):
+                    np.testing.assert_allclose(got, exp, rtol=1e-6, atol=1e-6, err_msg=str(act))
+                else:
+                    np.testing.assert_array_equal(got, exp, err_msg=str(act))
+    finally:
+        lib.dh_debug_force_splitk(0)
+
+
+@pytest.mark.parametrize("offset", [0, 1])
+@pytest.mark.parametrize("shape", [  # tile of the filter gradient
+    (9, 27, 19, 48, 3, 3, 80, 1),    # 128 x 128, 48 of 128 columns past the end
+    (9, 27, 19, 16, 3, 3, 64, 1),    # 128 x 64
+    (9, 27, 19, 16, 3, 3, 20, 1),    # 128 x 32
+    (9, 27, 19, 16, 2, 2, 64, 1),    # 64 x 64
+])
+def test_many_slices(A, shape, offset):
+    """Either side of the rule that lets eight threads share the slices of an output (64 of them), with counts that
+    eight does not divide; single and paired, against float64.  Tolerance: a sum of K products of magnitude below 1 in
+    32 bits, K * 2^-24 of its largest magnitude at the very worst, a hundredth of that here (rounding errors cancel)."""
+    import torch
+    print("shape", shape, "offset", offset, flush=True)
+    N, H, W, C, kh, kw, O, s = shape
+    (ph, Ho), (pw, Wo) = A.same_pad(H, kh, s), A.same_pad(W, kw, s)
+    lib, P = A.load(), torch.Tensor.data_ptr
+    ins = [rand_conv_inputs(seed, *shape)[::2] for seed in (7, 8)]
+    pad = torch.nn.functional.pad
+    exp = []
+    for x, dy in ins:
+        xp = pad(torch.from_numpy(x).double(), (0, 0, pw // 2, pw - pw // 2, ph // 2, ph - ph // 2)).numpy()
+        exp.append(np.stack([np.einsum("bijc,bijo->co", xp[:, i:i + Ho, j:j + Wo], dy.astype(np.float64), optimize=True)
+                             for i in range(kh) for j in range(kw)]).reshape(kh, kw, C, O))
+    dev = [(device(x), device(dy)) for x, dy in ins]
+    geom = (N, H, W, C, Ho, Wo, O, kh, kw, s, s, ph // 2, pw // 2)
+    tol = N * Ho * Wo * 2.0 ** -24
+    for splits in (63, 64, 100, 200):
+        lib.dh_debug_force_splitk(splits)
+        try:
+            d = room(kh * kw * C * O, offset)
+            A.check(lib.dh_conv2d_dk(P(dev[0][0]), P(dev[0][1]), P(d), *geom, None))
+            got = d.cpu().numpy().reshape(kh, kw, C, O)
+            np.testing.assert_allclose(got, exp[0], rtol=0, atol=tol, err_msg="%d splits" % splits)
+            again = room(kh * kw * C * O, offset)
+            A.check(lib.dh_conv2d_dk(P(dev[0][0]), P(dev[0][1]), P(again), *geom, None))
+            np.testing.assert_array_equal(got, again.cpu().numpy().reshape(kh, kw, C, O))
+            A.check(lib.dh_conv2d_dk_pair(P(dev[0][0]), P(dev[0][1]), P(dev[1][0]), P(dev[1][1]), P(d), *geom, None))
+            np.testing.assert_allclose(d.cpu().numpy().reshape(kh, kw, C, O), exp[0] + exp[1], rtol=0, atol=2 * tol,
+                                       err_msg="%d splits, pair" % splits)
+        finally:
+            lib.dh_debug_force_splitk(0)
