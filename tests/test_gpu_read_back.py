@@ -1,0 +1,66 @@
+"""Large copies to the host, which go through a ring of pinned chunks: every byte arrives, behind the work already queued, for
+lengths around the chunk and ring sizes, and from several threads at once."""
+import ctypes as C
+import threading
+
+import numpy as np
+import pytest
+import torch   # before the library: whichever comes first brings the HIP runtime that both use
+
+pytestmark = pytest.mark.gpu
+
+CHUNK, RING = 256 << 10, 4 << 20
+
+
+@pytest.fixture(scope="module")
+def A():
+    import __graft_entry__ as ge
+    A = ge.load_package().hipabi
+    A.check(A.load().dh_init(0))
+    return A
+
+
+def read(A, src, nbytes):
+    out = np.full(nbytes + 8, 0xa5, np.uint8)
+    A.check(A.load().dh_memcpy_d2h(C.c_void_p(out.ctypes.data + 4), C.c_void_p(src), C.c_size_t(nbytes)))
+    assert (out[:4] == 0xa5).all() and (out[-4:] == 0xa5).all()
+    return out[4:-4]
+
+
+@pytest.mark.parametrize("nbytes", [2 * CHUNK - 4, 2 * CHUNK, 2 * CHUNK + 4, 2 * CHUNK + 2, 1 << 20, RING - 4, RING, RING + 4,
+                                    RING + CHUNK + 16, 3 * RING + 12, 13 << 20])
+@pytest.mark.parametrize("offset", [0, 4, 16])
+def test_lengths(A, nbytes, offset):
+    print("bytes", nbytes, "offset", offset, flush=True)
+    a = torch.randint(0, 256, (nbytes + 64,), dtype=torch.uint8, device="cuda")
+    exp = a.cpu().numpy()
+    for _ in range(2):
+        np.testing.assert_array_equal(read(A, a.data_ptr() + offset, nbytes), exp[offset:offset + nbytes])
+
+
+def test_behind_queued_work(A):
+    a = torch.zeros(3 << 20, device="cuda")
+    for i in range(5):
+        b = a
+        for _ in range(20):
+            b = b + 1
+        a = b
+        got = read(A, a.data_ptr(), a.numel() * 4).view(np.float32)
+        assert (got == 20 * (i + 1)).all()
+
+
+def test_threads(A):
+    srcs = [torch.full((700000 + 1000 * i,), float(i + 1), device="cuda") for i in range(4)]
+    torch.cuda.synchronize()
+    bad = []
+
+    def work(i):
+        for _ in range(6):
+            if not (read(A, srcs[i].data_ptr(), srcs[i].numel() * 4).view(np.float32) == i + 1).all():
+                bad.append(i)
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(4)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not bad
