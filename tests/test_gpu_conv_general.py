@@ -57,3 +57,17 @@ def test_general_kernel(be, orc64, shape, splits):
         err = np.abs(got[op].astype(np.float64) - exact[op].astype(np.float64))
         assert got[op].shape == exact[op].shape, op
         assert (err <= bound).all(), (op, float((err / bound).max()))
+
+
+@pytest.mark.parametrize("splits", [1, 2, 3])
+@pytest.mark.parametrize("channels", [5, 17, 33, 49, 65, 97])
+def test_slabs_in_flight(be, orc64, channels, splits):
+    """Contractions of 1, 2, 3, 4, 5 and 7 slabs (forward; input gradient two more channels), whole and in shares of one slab and more:
+    the two slabs that are loaded ahead may lie past the share or past the end."""
+    test_general_kernel(be, orc64, (2, 6, 7, channels, 1, 1, channels + 2, 1), splits)
+
+
+@pytest.mark.parametrize("shape", [(2, 9, 7, 18, 4, 4, 30, 2), (26, 10, 10, 30, 5, 5, 3, 2), (40, 16, 16, 18, 4, 4, 30, 1)])
+def test_shares_of_four_and_eight_slabs(be, orc64, shape):
+    """Either side of the rule for the smallest share, with the library's own choice of the split."""
+    test_general_kernel(be, orc64, shape, 0)
