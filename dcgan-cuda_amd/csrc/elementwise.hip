@@ -201,24 +201,39 @@ struct ActGrad
 {
     int act;
     float alpha;
-    __device__ float operator()(float ref, float d) const
+};
+
+// The gradients of the piecewise linear activations and of the other two, without a branch: a switch in the row loop kept
+// the loads of a row behind the arithmetic of the one before.  Measured, 16384 x 128 elements 6.7 -> 6.2 us; forward and backward
+// pass of 23 layers 0.9 % less in the mean.
+struct LinearGrad
+{
+    bool relu;
+    float alpha;
+    __host__ __device__ explicit LinearGrad(ActGrad g) : relu(g.act == DH_ACT_RELU), alpha(g.act == DH_ACT_LEAKY ? g.alpha : 1.f) {}
+    __device__ __forceinline__ float operator()(float ref, float d) const
     {
-        switch (act)
-        {
-        case DH_ACT_RELU: return ref > 0.f ? d : 0.f;
-        case DH_ACT_LEAKY: return ref < 0.f ? alpha * d : d;
-        case DH_ACT_TANH: return (1.f - ref * ref) * d;
-        case DH_ACT_SIGMOID: return ref * (1.f - ref) * d;
-        default: return d;
-        }
+        const bool through = relu ? ref > 0.f : !(ref < 0.f);
+        const float below = relu ? 0.f : alpha * d;
+        return through ? d : below;
+    }
+};
+struct SmoothGrad
+{
+    bool tanh;
+    __host__ __device__ explicit SmoothGrad(ActGrad g) : tanh(g.act == DH_ACT_TANH) {}
+    __device__ __forceinline__ float operator()(float ref, float d) const
+    {
+        const float slope = tanh ? 1.f - ref * ref : ref * (1.f - ref);
+        return slope * d;
     }
 };
 
-template <bool FUSED>
+template <bool FUSED, class Grad>
 __global__ __launch_bounds__(TPB) void colsum_stage1(const float* __restrict__ a, const float* __restrict__ act_ref,
                                                      float* __restrict__ dz, float* __restrict__ partial,
                                                      size_t rows, uint32_t cols, uint32_t G, size_t rows_per_chunk,
-                                                     ActGrad g)
+                                                     Grad g)
 {
     __shared__ float lds[TPB];
     const uint32_t t = threadIdx.x;
@@ -284,11 +299,11 @@ __global__ __launch_bounds__(TPB) void colsum_stage1(const float* __restrict__ a
 // accessed one by one), G4 = 256 / (cols / 4) rows lie side by side for matrices of up to 1024
 // columns, wider ones are cut into tiles of 1024 columns.  Same two-level order of additions as the
 // scalar kernel: a lane adds its rows serially, lanes of the same columns are added in lane order.
-template <bool FUSED, bool ALIGNED>
+template <bool FUSED, bool ALIGNED, class Grad>
 __global__ __launch_bounds__(TPB) void colsum_stage1_v4(const float* __restrict__ a, const float* __restrict__ act_ref,
                                                         float* __restrict__ dz, float* __restrict__ partial,
                                                         size_t rows, uint32_t cols, uint32_t G4, size_t rows_per_chunk,
-                                                        ActGrad g)
+                                                        Grad g)
 {
     __shared__ float4 lds[TPB];
     const uint32_t t = threadIdx.x;
@@ -471,15 +486,21 @@ int run_colsum(const char* who, const float* a, const float* act_ref, float* dz,
     ProfScope prof(fused ? "hbm:activation gradient + column sums (12 B/elem)" : "hbm:column sums (4 B/elem)",
                    (fused ? 12.0 : 4.0) * rows * cols, st, fixed_scratch ? 1 << 20 : 2);   // no events without allocating
     const bool al = aligned16(a) && (!fused || (aligned16(act_ref) && aligned16(dz)));
-#define DH_COLSUM_LAUNCH(KERNEL) \
-    hipLaunchKernelGGL(KERNEL, grid, dim3(TPB), 0, st, a, act_ref, dz, partial, rows, (uint32_t)cols, cut.G, cut.rows_per_chunk, g)
-    if (cut.vec4 && fused && al) DH_COLSUM_LAUNCH((colsum_stage1_v4<true, true>));
-    else if (cut.vec4 && fused) DH_COLSUM_LAUNCH((colsum_stage1_v4<true, false>));
-    else if (cut.vec4 && al) DH_COLSUM_LAUNCH((colsum_stage1_v4<false, true>));
-    else if (cut.vec4) DH_COLSUM_LAUNCH((colsum_stage1_v4<false, false>));
-    else if (fused) DH_COLSUM_LAUNCH(colsum_stage1<true>);
-    else DH_COLSUM_LAUNCH(colsum_stage1<false>);
-#undef DH_COLSUM_LAUNCH
+    auto launch = [&](auto kernel, auto grad) {
+        hipLaunchKernelGGL(kernel, grid, dim3(TPB), 0, st, a, act_ref, dz, partial, rows, (uint32_t)cols, cut.G, cut.rows_per_chunk, grad);
+    };
+    auto fused_launch = [&](auto grad) {
+        using Grad = decltype(grad);
+        if (cut.vec4 && al) launch(colsum_stage1_v4<true, true, Grad>, grad);
+        else if (cut.vec4) launch(colsum_stage1_v4<true, false, Grad>, grad);
+        else launch(colsum_stage1<true, Grad>, grad);
+    };
+    const LinearGrad linear(g);
+    if (fused && (g.act == DH_ACT_TANH || g.act == DH_ACT_SIGMOID)) fused_launch(SmoothGrad(g));
+    else if (fused) fused_launch(linear);
+    else if (cut.vec4 && al) launch(colsum_stage1_v4<false, true, LinearGrad>, linear);
+    else if (cut.vec4) launch(colsum_stage1_v4<false, false, LinearGrad>, linear);
+    else launch(colsum_stage1<false, LinearGrad>, linear);
     DH_LAUNCH_CHECK(who);
     if (db && !parts_out && !single)
     {
