@@ -115,3 +115,27 @@ def test_many_slices(A, shape, offset):
                                        err_msg="%d splits, pair" % splits)
         finally:
             lib.dh_debug_force_splitk(0)
+
+
+@pytest.mark.parametrize("shape", [  # either side of the rule for the smallest share of a small launch
+    (4, 16, 16, 64, 3, 3, 64, 1),    # shares of 4 slabs, 9 slices
+    (1, 16, 16, 80, 4, 4, 64, 1),    # 80 slabs, 20 slices
+    (1, 16, 16, 96, 4, 4, 64, 1),    # 96 slabs: shares of 8
+    (9, 16, 16, 80, 4, 4, 144, 1),   # 18 x 80 slabs and more: shares of 8
+])
+def test_small_launches(A, shape):
+    """Forward product and input gradient with the library's own split against the same launch cut differently (one slice):
+    two orders of the sums differ by at most n 2^-24 of the sum of the magnitudes, here bounded by that of the largest."""
+    print("shape", shape, flush=True)
+    be = A.HipBackend(0)
+    N, H, W, C, kh, kw, O, s = shape
+    x, k, dy = rand_conv_inputs(9, *shape)
+    got = be.conv2d(x, k, (s, s)), be.conv2d_input_grad(dy, k, s, (H, W))
+    mag = be.conv2d(np.abs(x), np.abs(k), (s, s)), be.conv2d_input_grad(np.abs(dy), np.abs(k), s, (H, W))
+    be.lib.dh_debug_force_splitk(1)
+    try:
+        whole = be.conv2d(x, k, (s, s)), be.conv2d_input_grad(dy, k, s, (H, W))
+    finally:
+        be.lib.dh_debug_force_splitk(0)
+    for g, w, m, n in zip(got, whole, mag, (kh * kw * C, kh * kw * O)):
+        assert np.abs(g - w).max() <= 2.0 ** -24 * n * m.max()
