@@ -3,6 +3,7 @@
 #include "dh_common.h"
 
 #include <atomic>
+#include <condition_variable>
 #include <cstdarg>
 #include <cstdio>
 #include <cstring>
@@ -215,6 +216,8 @@ struct Read
     std::atomic<int> next{0};                       // next chunk to take out
     std::atomic<bool> stop{false};                  // after an error: no further chunk will arrive
     std::atomic<int> taken[READ_SLOTS] = {};        // chunks taken out of the slot so far
+    std::mutex mu;                                  // with `moved`: helpers sleep until the first chunk is there, however long the
+    std::condition_variable moved;                  // work in front of the copy takes; the chunks after it are microseconds apart
 
     size_t begin(int c) const { return (size_t)c * READ_CHUNK; }
     size_t size(int c) const { return begin(c) + READ_CHUNK <= bytes ? READ_CHUNK : bytes - begin(c); }
@@ -224,8 +227,21 @@ struct Read
         memcpy(dst + begin(c), ring + (size_t)(c % READ_SLOTS) * READ_CHUNK, size(c));
         taken[c % READ_SLOTS].fetch_add(1, std::memory_order_release);
     }
+    template <class T>
+    void announce(std::atomic<T>& what, T value)
+    {
+        {
+            std::lock_guard<std::mutex> lock(mu);
+            what.store(value, std::memory_order_release);
+        }
+        moved.notify_all();
+    }
     void help()
     {
+        {
+            std::unique_lock<std::mutex> lock(mu);
+            moved.wait(lock, [this] { return arrived.load() > 0 || stop.load(); });
+        }
         for (int c = next.fetch_add(1); c < chunks; c = next.fetch_add(1))
         {
             while (arrived.load(std::memory_order_acquire) <= c)
@@ -298,6 +314,8 @@ int read_staged(DeviceState& st, char* dst, const char* src, size_t bytes)
             break;
         if (helpers == 0)
             r.take(c);
+        else if (c == 0)
+            r.announce(r.arrived, 1);
         else
             r.arrived.store(c + 1, std::memory_order_release);
         // refill the slots that have been emptied; with all others in flight, wait for the oldest
@@ -315,7 +333,7 @@ int read_staged(DeviceState& st, char* dst, const char* src, size_t bytes)
     if (err != hipSuccess)
     {
         (void)hipStreamSynchronize(nullptr);    // no copy into the ring outlives the call
-        r.stop.store(true, std::memory_order_release);
+        r.announce(r.stop, true);
     }
     for (int h = 0; h < helpers; ++h)
         helper[h].join();
