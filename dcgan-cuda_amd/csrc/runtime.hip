@@ -186,13 +186,16 @@ bool known_to_device(const void* ptr)
     return attr.type != hipMemoryTypeUnregistered;
 }
 
-// Whether [ptr, ptr + bytes) lies within one allocation on the device.
-bool inside_device_memory(const void* ptr, size_t bytes)
+// Whether [ptr, ptr + bytes) lies within one allocation on `device`, and that is also the device of the calling thread: kernels and
+// events go to the null stream of the thread's device (HIP keeps one a thread), which other devices' memory and work know nothing of.
+bool inside_memory_of(int device, const void* ptr, size_t bytes)
 {
     hipPointerAttribute_t attr;
     void* base = nullptr;
     size_t size = 0;
-    if (hipPointerGetAttributes(&attr, ptr) != hipSuccess || attr.type != hipMemoryTypeDevice ||
+    int current = -1;
+    if (hipGetDevice(&current) != hipSuccess || current != device || hipPointerGetAttributes(&attr, ptr) != hipSuccess ||
+        attr.type != hipMemoryTypeDevice || attr.device != device ||
         hipMemGetAddressRange(&base, &size, const_cast<void*>(ptr)) != hipSuccess)
     {
         (void)hipGetLastError();
@@ -458,14 +461,16 @@ int dh_memcpy_d2h(void* dst, const void* src, size_t bytes)
     // Measured: a stretch of six training iterations at batch 64 that ends with reading all weights (38 MB in 18 pieces) 20.5 -> 17.9 ms,
     // sampling 64 images (3.1 MB) 445 -> 395 us.  Below 512 KiB the copy is one round trip either way.
     // Small ones, a copy while another is in progress, host memory that the device reaches by itself (pinned, managed) and
-    // whatever is not inside one device allocation take the runtime's copy, which refuses what it always did.
+    // whatever is not inside one allocation on the library's device, that being the thread's too, take the runtime's copy, which finds
+    // the device of the memory by itself and refuses what it always did.
+    const int device = g_cur;   // once: another thread may call dh_init meanwhile
     if (dst && bytes >= READ_STAGED_MIN && (reinterpret_cast<uintptr_t>(src) & 15) == 0 && bytes % 4 == 0 && !known_to_device(dst) &&
-        inside_device_memory(src, bytes))
+        inside_memory_of(device, src, bytes))
     {
         std::unique_lock<std::mutex> ring(g_read_mu, std::try_to_lock);
         if (ring.owns_lock())
         {
-            const int rc = read_staged(g_dev[g_cur], static_cast<char*>(dst), static_cast<const char*>(src), bytes);
+            const int rc = read_staged(g_dev[device], static_cast<char*>(dst), static_cast<const char*>(src), bytes);
             if (rc != READ_NOT_STARTED)
                 return rc;
         }
