@@ -470,6 +470,11 @@ int dh_memcpy_d2h(void* dst, const void* src, size_t bytes)
         std::unique_lock<std::mutex> ring(g_read_mu, std::try_to_lock);
         if (ring.owns_lock())
         {
+            // While a stream is captured the runtime refuses a blocking copy, one of no bytes too (1.3 us); the ring's launches it
+            // would take.
+            const hipError_t allowed = hipMemcpy(dst, src, 0, hipMemcpyDeviceToHost);
+            if (allowed != hipSuccess)
+                return fail_hip(allowed, "hipMemcpy(dst, src, bytes, hipMemcpyDeviceToHost)");
             const int rc = read_staged(g_dev[device], static_cast<char*>(dst), static_cast<const char*>(src), bytes);
             if (rc != READ_NOT_STARTED)
                 return rc;

@@ -1,6 +1,6 @@
 // A HIP runtime of two devices in host memory, as far as reading back needs it (test infrastructure): loaded in front of the real
 // one by tests/test_read_back_route.py.  "Device memory" is host memory that the test has declared; the current device is the calling
-// thread's; an event belongs to the device that was current when it was made, and recording it from another is an error.
+// thread's; while a stream is captured a blocking copy is refused, whatever its size; an event belongs to the device that was current when it was made, and recording it from another is an error.
 #include <hip/hip_runtime_api.h>
 
 #include <atomic>
@@ -16,7 +16,7 @@ std::mutex mu;
 std::vector<Range> ranges;
 thread_local int current = 0;
 thread_local hipError_t last = hipSuccess;   // of a launch
-std::atomic<int> launches{0}, copies{0}, fail_launch{-1}, fail_pinned{0};
+std::atomic<int> launches{0}, copies{0}, fail_launch{-1}, fail_pinned{0}, captured{0};
 char symbol[256];
 
 bool find(const void* p, Range* out)
@@ -51,6 +51,7 @@ void fake_reset(int launch_that_fails, int no_pinned_memory)
     fail_launch = launch_that_fails;
     fail_pinned = no_pinned_memory;
 }
+void fake_capture(int on) { captured = on; }
 int fake_launches() { return launches; }
 int fake_copies() { return copies; }
 
@@ -110,7 +111,8 @@ hipError_t hipEventSynchronize(hipEvent_t) { return hipSuccess; }
 hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
 hipError_t hipMemcpy(void* dst, const void* src, size_t bytes, hipMemcpyKind)
 {
-    ++copies;
+    if (captured) return hipErrorStreamCaptureImplicit;
+    copies += bytes > 0;
     if (!dst || !src) return hipErrorInvalidValue;
     memcpy(dst, src, bytes);
     return hipSuccess;

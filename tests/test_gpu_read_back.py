@@ -64,3 +64,20 @@ def test_threads(A):
     for t in threads:
         t.join()
     assert not bad
+
+
+@pytest.mark.parametrize("nbytes", [64 << 10, 5 << 20])
+def test_refused_while_a_stream_is_captured(A, nbytes):
+    """As the blocking copy is, whatever the size and whether the ring is there already."""
+    lib, st, graph = A.load(), C.c_void_p(), C.c_void_p()
+    src = torch.full((nbytes // 4,), 3.0, device="cuda")
+    out = np.zeros(nbytes // 4, np.float32)
+    assert lib.hipStreamCreateWithFlags(C.byref(st), 1) == 0    # kept: a stream whose capture was ended by an error cannot be waited for
+    for _ in range(2):
+        torch.cuda.synchronize()
+        assert lib.hipStreamBeginCapture(st, 0) == 0
+        rc = lib.dh_memcpy_d2h(C.c_void_p(out.ctypes.data), C.c_void_p(src.data_ptr()), C.c_size_t(nbytes))
+        lib.hipStreamEndCapture(st, C.byref(graph))             # an error too
+        lib.hipGetLastError()
+        assert rc != 0 and (out == 0).all()
+        assert (read(A, src.data_ptr(), nbytes).view(np.float32) == 3.0).all()

@@ -102,6 +102,17 @@ assert lib.dh_memcpy_d2h(None, C.c_void_p(a.ctypes.data), C.c_size_t(a.size)) !=
 assert lib.dh_memcpy_d2h(C.c_void_p(a.ctypes.data), None, C.c_size_t(a.size)) != 0
 assert fake.fake_launches() == 0 and fake.fake_copies() == 2
 """,
+    "a stream is captured": """
+lib.dh_init(0)
+a, small = memory(5 * MB), memory(4096)
+for i in range(2):
+    fake.fake_capture(1)
+    read(small, rc=1)
+    expect(read(a, rc=1), "both or none")
+    fake.fake_capture(0)
+    expect(read(a), "ring")
+    expect(read(small), "runtime")
+""",
     "errors on the way": """
 lib.dh_init(0)
 a = memory(9 * MB)
