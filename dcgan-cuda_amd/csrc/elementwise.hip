@@ -204,11 +204,13 @@ struct ActGrad
 };
 
 // The gradients of the piecewise linear activations and of the other two, without a branch: a switch in the row loop kept
-// the loads of a row behind the arithmetic of the one before.  Measured, 16384 x 128 elements 6.7 -> 6.2 us; forward and backward
-// pass of 23 layers 0.9 % less in the mean.
+// the loads of a row behind the arithmetic of the one before.  Measured, with the second stage, switch / without: leaky relu 16384 x 128
+// 8.6 / 8.0 us, 65536 x 64 13.4 / 13.2; tanh 16384 x 128 8.4 / 7.8, 262144 x 3 6.6 / 6.6.
+// The flags are ints: a bool member of an argument is a byte that the compiler did not promote to a register but kept in LDS, a byte per
+// thread, and read for every element (tanh 16384 x 128 20.5 us, 262144 x 3 19.2).
 struct LinearGrad
 {
-    bool relu;
+    int relu;
     float alpha;
     __host__ __device__ explicit LinearGrad(ActGrad g) : relu(g.act == DH_ACT_RELU), alpha(g.act == DH_ACT_LEAKY ? g.alpha : 1.f) {}
     __device__ __forceinline__ float operator()(float ref, float d) const
@@ -220,7 +222,7 @@ struct LinearGrad
 };
 struct SmoothGrad
 {
-    bool tanh;
+    int tanh;
     __host__ __device__ explicit SmoothGrad(ActGrad g) : tanh(g.act == DH_ACT_TANH) {}
     __device__ __forceinline__ float operator()(float ref, float d) const
     {

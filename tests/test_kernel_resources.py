@@ -1,0 +1,53 @@
+"""What the compiler makes of the kernels, read from its assembly: no variable that should be a register ends up in memory.
+Without a GPU."""
+import concurrent.futures
+import glob
+import importlib.util
+import os
+import re
+import subprocess
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+
+
+def build_module():
+    spec = importlib.util.spec_from_file_location("build_flags", os.path.join(ROOT, "dcgan-cuda_amd", "build.py"))
+    mod = importlib.util.module_from_spec(spec)
+    spec.loader.exec_module(mod)
+    return mod
+
+
+@pytest.fixture(scope="module")
+def assembly(tmp_path_factory):
+    """{source: assembly text}"""
+    b = build_module()
+    if not os.path.exists(b.HIPCC):
+        pytest.skip("hipcc not found")
+    out = tmp_path_factory.mktemp("asm")
+
+    def one(src):
+        name = os.path.basename(src)
+        s = str(out / (name + ".s"))
+        subprocess.run([b.HIPCC] + b.HIPFLAGS + ["--cuda-device-only", "-S", src, "-o", s], check=True, capture_output=True)
+        return name, open(s).read()
+    with concurrent.futures.ThreadPoolExecutor(8) as ex:
+        return dict(ex.map(one, sorted(glob.glob(os.path.join(b.CSRC, "*.hip")))))
+
+
+def kernels(text):
+    """(name, descriptor directives as a dict) of every kernel"""
+    for m in re.finditer(r"\.amdhsa_kernel (\S+)(.*?)\.end_amdhsa_kernel", text, re.S):
+        yield m.group(1), dict(re.findall(r"\.amdhsa_(\S+) (\S+)", m.group(2)))
+
+
+def test_no_variable_in_lds(assembly):
+    """A local variable that the compiler cannot keep in a register and moves to LDS is indexed by the workgroup's extents, which
+    it reads from the dispatch packet: the one use of that pointer here, no kernel asks for its extents."""
+    count = 0
+    for src, text in assembly.items():
+        for name, d in kernels(text):
+            count += 1
+            assert d["user_sgpr_dispatch_ptr"] == "0", (src, name)
+    assert count > 100
