@@ -515,6 +515,21 @@ def test_paired_launches(be, orc, shape):
     close(dk, exp.astype(np.float32), scale=max(1.0, float(np.abs(exp).max())), what="paired filter gradient")
 
 
+@pytest.mark.parametrize("splits", [0, 1, 3])     # 1: a share runs from the first instance's operands into the second's
+@pytest.mark.parametrize("shape", [  # tile of the filter gradient
+    (37, 16, 16, 48, 5, 5, 80, 2),    # 128 x 128
+    (37, 8, 8, 32, 3, 3, 64, 1),      # 128 x 64
+    (37, 9, 7, 16, 3, 3, 32, 1),      # 128 x 32
+    (37, 8, 8, 16, 2, 2, 48, 1),      # 64 x 64
+])
+def test_paired_launches_at_a_batch_that_is_no_multiple_of_16(be, orc, shape, splits):
+    be.lib.dh_debug_force_splitk(splits)
+    try:
+        test_paired_launches(be, orc, shape)
+    finally:
+        be.lib.dh_debug_force_splitk(0)
+
+
 @pytest.mark.parametrize("shape", [(64, 32, 32, 64, 5, 5, 128, 2), (64, 16, 16, 128, 5, 5, 256, 2), (64, 8, 8, 256, 5, 5, 512, 2)])
 def test_paired_launches_at_batch_64_match_the_single_launches(be, shape):
     """At the benchmark's shapes, on inputs in the benchmark's distributions, with a fused epilogue: the

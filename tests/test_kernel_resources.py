@@ -51,3 +51,21 @@ def test_no_variable_in_lds(assembly):
             count += 1
             assert d["user_sgpr_dispatch_ptr"] == "0", (src, name)
     assert count > 100
+
+
+def test_no_spills(assembly):
+    """No kernel keeps registers in memory."""
+    for src, text in assembly.items():
+        spills = dict(zip(re.findall(r"\.symbol:\s*(\S+)", text), re.findall(r"\.vgpr_spill_count:\s*(\d+)", text)))
+        for name, d in kernels(text):
+            assert d["private_segment_fixed_size"] == "0" and spills.get(name + ".kd", spills.get("'" + name + ".kd'")) == "0", (src, name)
+
+
+def test_no_loop_around_a_load(assembly):
+    """The address of a buffer is the same for all lanes: where the compiler cannot tell, it puts a loop over the lanes around the
+    load, which ends in a branch on the lanes left."""
+    for src, text in assembly.items():
+        for name, body in re.findall(r"^(\S*conv_igemm_fast\S*):(.*?)s_endpgm", text, re.S | re.M):
+            lines = [l.split()[0] for l in body.split("\n") if l.startswith("\t") and l.split()]
+            loops = sum(l.startswith("buffer_load") and "s_cbranch_execnz" in lines[i:i + 4] for i, l in enumerate(lines))
+            assert loops == 0, (src, name, loops)
