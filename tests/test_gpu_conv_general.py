@@ -71,3 +71,21 @@ def test_slabs_in_flight(be, orc64, channels, splits):
 def test_shares_of_four_and_eight_slabs(be, orc64, shape):
     """Either side of the rule for the smallest share, with the library's own choice of the split."""
     test_general_kernel(be, orc64, shape, 0)
+
+
+@pytest.mark.parametrize("splits", [1, 2])
+@pytest.mark.parametrize("channels", [49, 65, 97, 113, 145, 289])
+def test_register_sets(be, orc64, channels, splits):
+    """Shares of 2 to 19 slabs, odd and even, on either side of the rule for the second register set (more than 4, input gradient more
+    than 6); on all tile shapes."""
+    for out in (5, 37, 66):
+        test_general_kernel(be, orc64, (2, 3, 5, channels, 1, 1, out, 1), splits)      # filter gradient: 2 slabs
+        test_general_kernel(be, orc64, (2, 3, 5, out, 1, 1, channels, 1), splits)
+    test_general_kernel(be, orc64, (2, 6 + channels % 3, 7, 17, 1, 1, 70, 1), splits)  # 6, 7 and 8 slabs
+    test_general_kernel(be, orc64, (5, 6, 5, channels, 1, 1, 37, 1), splits)           # 10 slabs
+
+
+@pytest.mark.parametrize("channels", [99, 131])
+def test_register_sets_with_many_workgroups(be, orc64, channels):
+    """More than two workgroups per unit: one set for 7 slabs, two for 9."""
+    test_general_kernel(be, orc64, (40, 41, 41, channels, 1, 1, 3, 1), 1)

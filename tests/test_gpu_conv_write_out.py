@@ -82,8 +82,8 @@ def test_activations(A, shape, splits, offset):
     (9, 27, 19, 16, 2, 2, 64, 1),    # 64 x 64
 ])
 def test_many_slices(A, shape, offset):
-    """Either side of the rule that lets eight threads share the slices of an output (64 of them), with counts that
-    eight does not divide; single and paired, against float64.  Tolerance: a partial sum of K products of numbers
+    """One thread an output and eight sharing its slices (58, 97 and 145 of them, 193 paired: counts that eight does not
+    divide), every tile with the same number; single and paired, against float64.  Tolerance: a partial sum of K products of numbers
     in (-1, 1) is about sqrt(K) / 3, each of up to K roundings at most 2^-25 of that, and they add up as their root:
     K / 3 * 2^-25, taken six times."""
     print("shape", shape, "offset", offset, flush=True)
@@ -139,3 +139,77 @@ def test_small_launches(A, shape):
         be.lib.dh_debug_force_splitk(0)
     for g, w, m, n in zip(got, whole, mag, (kh * kw * C, kh * kw * O)):
         assert np.abs(g - w).max() <= 2.0 ** -24 * n * m.max()
+
+
+def filter_gradient_float64(A, x, dy, kh, kw, s):
+    N, H, W, C = x.shape
+    _, Ho, Wo, O = dy.shape
+    ph, pw = A.same_pad(H, kh, s)[0], A.same_pad(W, kw, s)[0]
+    xp = np.pad(x.astype(np.float64), ((0, 0), (ph // 2, ph - ph // 2), (pw // 2, pw - pw // 2), (0, 0)))
+    return np.stack([np.einsum("bijc,bijo->co", xp[:, i:i + Ho * s:s, j:j + Wo * s:s][:, :Ho, :Wo], dy.astype(np.float64), optimize=True)
+                     for i in range(kh) for j in range(kw)]).reshape(kh, kw, C, O)
+
+
+@pytest.mark.parametrize("shape", [
+    # one slab a slice, as many slices as slabs: 63, 64 and 65 of them, the bound of the sharing between the first two
+    (9, 14, 8, 48, 3, 3, 80, 1),
+    (8, 16, 8, 48, 3, 3, 80, 1),
+    (5, 16, 13, 48, 3, 3, 80, 1),
+    # 62 and 64 of them in the paired launch, which has twice the slabs
+    (8, 31, 2, 48, 3, 3, 80, 1),
+    (8, 16, 4, 48, 3, 3, 80, 1),
+    # a tile is one tap, whose pixels outside the image are left out: 81 slices in the middle, 25 in the corners, where some of
+    # the eight threads have none
+    (16, 9, 9, 128, 9, 9, 32, 1),
+])
+def test_shared_slices_at_the_bound(A, shape):
+    """Tolerance as in test_many_slices."""
+    print("shape", shape, flush=True)
+    N, H, W, C, kh, kw, O, s = shape
+    (ph, Ho), (pw, Wo) = A.same_pad(H, kh, s), A.same_pad(W, kw, s)
+    lib, P = A.load(), torch.Tensor.data_ptr
+    ins = [rand_conv_inputs(seed, *shape)[::2] for seed in (7, 8)]
+    exp = [filter_gradient_float64(A, x, dy, kh, kw, s) for x, dy in ins]
+    dev = [(device(x), device(dy)) for x, dy in ins]
+    geom = (N, H, W, C, Ho, Wo, O, kh, kw, s, s, ph // 2, pw // 2)
+    tol = N * Ho * Wo * 2.0 ** -24
+    lib.dh_debug_force_splitk(200)
+    try:
+        d = room(kh * kw * C * O, 0)
+        A.check(lib.dh_conv2d_dk(P(dev[0][0]), P(dev[0][1]), P(d), *geom, None))
+        np.testing.assert_allclose(d.cpu().numpy().reshape(kh, kw, C, O), exp[0], rtol=0, atol=tol)
+        A.check(lib.dh_conv2d_dk_pair(P(dev[0][0]), P(dev[0][1]), P(dev[1][0]), P(dev[1][1]), P(d), *geom, None))
+        np.testing.assert_allclose(d.cpu().numpy().reshape(kh, kw, C, O), exp[0] + exp[1], rtol=0, atol=2 * tol)
+    finally:
+        lib.dh_debug_force_splitk(0)
+
+
+@pytest.mark.parametrize("shape", [  # as in test_small_launches, and a launch of position-major rows
+    (4, 16, 16, 64, 3, 3, 64, 1),
+    (1, 16, 16, 80, 4, 4, 64, 1),
+    (16, 4, 4, 64, 5, 5, 128, 2),
+])
+def test_small_paired_launches(A, shape):
+    """Two instances in one launch against the single launches cut into one slice each; bound as in test_small_launches."""
+    print("shape", shape, flush=True)
+    be = A.HipBackend(0)
+    N, H, W, C, kh, kw, O, s = shape
+    (ph, Ho), (pw, Wo) = A.same_pad(H, kh, s), A.same_pad(W, kw, s)
+    lib, P = A.load(), torch.Tensor.data_ptr
+    ins = [rand_conv_inputs(seed, *shape) for seed in (9, 10)]
+    k = ins[0][1]
+    kd, xd, dyd = device(k), [device(x) for x, _, _ in ins], [device(dy) for _, _, dy in ins]
+    y, dx = [torch.empty_like(t) for t in dyd], [torch.empty_like(t) for t in xd]
+    fwd = (N, H, W, C, kh, kw, O, s, s, ph // 2, pw // 2, Ho, Wo)
+    adj = (N, Ho, Wo, O, kh, kw, C, s, s, ph // 2, pw // 2, H, W)
+    A.check(lib.dh_conv2d_fwd_pair(P(xd[0]), P(xd[1]), P(kd), P(y[0]), P(y[1]), *fwd, None, A.ACT_NONE, 0.0, None))
+    A.check(lib.dh_conv2d_dx_pair(P(dyd[0]), P(dyd[1]), P(kd), P(dx[0]), P(dx[1]), *adj, None, A.ACT_NONE, 0.0, None))
+    for i, (x, _, dy) in enumerate(ins):
+        mag = be.conv2d(np.abs(x), np.abs(k), (s, s)), be.conv2d_input_grad(np.abs(dy), np.abs(k), s, (H, W))
+        lib.dh_debug_force_splitk(1)
+        try:
+            whole = be.conv2d(x, k, (s, s)), be.conv2d_input_grad(dy, k, s, (H, W))
+        finally:
+            lib.dh_debug_force_splitk(0)
+        for g, w, m, n in zip((y[i].cpu().numpy(), dx[i].cpu().numpy()), whole, mag, (kh * kw * C, kh * kw * O)):
+            assert np.abs(g - w).max() <= 2.0 ** -24 * n * m.max()

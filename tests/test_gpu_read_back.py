@@ -67,6 +67,15 @@ def test_threads(A):
 
 
 @pytest.mark.parametrize("nbytes", [64 << 10, 5 << 20])
+def test_into_pinned_memory(A, nbytes):
+    """The runtime's way, whatever the size."""
+    src = torch.arange(nbytes // 4, device="cuda", dtype=torch.float32)
+    out = torch.empty(nbytes // 4, pin_memory=True)
+    A.check(A.load().dh_memcpy_d2h(C.c_void_p(out.data_ptr()), C.c_void_p(src.data_ptr()), C.c_size_t(nbytes)))
+    assert torch.equal(out, torch.arange(nbytes // 4, dtype=torch.float32))
+
+
+@pytest.mark.parametrize("nbytes", [64 << 10, 5 << 20])
 def test_refused_while_a_stream_is_captured(A, nbytes):
     """As the blocking copy is, whatever the size and whether the ring is there already."""
     lib, st, graph = A.load(), C.c_void_p(), C.c_void_p()
