@@ -24,7 +24,7 @@ __attribute__((used)) static __device__ __align__(256) unsigned char scratch[STA
 // Chunks of a large copy to the host, see dh_memcpy_d2h.
 constexpr size_t READ_CHUNK = 256 * 1024;
 constexpr int READ_SLOTS = 16;
-constexpr size_t READ_STAGED_MIN = 512 * 1024;
+constexpr size_t READ_STAGED_MIN = 2 * 1024 * 1024;   // smaller ones gain nothing
 constexpr int READ_THREADS_MAX = 3;
 
 struct DeviceState
@@ -297,8 +297,7 @@ int read_staged(DeviceState& st, char* dst, const char* src, size_t bytes)
 
     std::thread helper[READ_THREADS_MAX];
     int helpers = 0;
-    const int wanted = (int)(bytes / (READ_STAGED_MIN * 2));
-    while (err == hipSuccess && helpers < READ_THREADS_MAX && helpers < wanted)
+    while (err == hipSuccess && helpers < READ_THREADS_MAX && helpers < (int)(bytes >> 20))
     {
         try
         {
@@ -459,7 +458,9 @@ int dh_memcpy_d2h(void* dst, const void* src, size_t bytes)
     // the host empties the ones that are there, with helper threads, since the page faults and the copy of one thread are
     // slower than the bus.  The runtime's own copy into pageable memory takes turns: a chunk across the bus, a wait, its copy.
     // Measured: a stretch of six training iterations at batch 64 that ends with reading all weights (38 MB in 18 pieces) 20.5 -> 17.9 ms,
-    // sampling 64 images (3.1 MB) 445 -> 395 us.  Below 512 KiB the copy is one round trip either way.
+    // sampling 64 images (3.1 MB) 445 -> 395 us.  From 2 MiB on, where two helpers pay: runtime / ring, us, 2 MiB 119 / 98, 4 MiB 230 / 176,
+    // 13 MiB 717 / 505.  With one helper, which does all the copying while the caller waits, or with none the ring gained nothing: 512 KiB
+    // 29.9 / 31.9, 1 MiB 58 / 61, 1.75 MiB 102 / 103 (medians).
     // Small ones, a copy while another is in progress, host memory that the device reaches by itself (pinned, managed) and
     // whatever is not inside one allocation on the library's device, that being the thread's too, take the runtime's copy, which finds
     // the device of the memory by itself and refuses what it always did.

@@ -27,7 +27,8 @@ def read(A, src, nbytes):
     return out[4:-4]
 
 
-@pytest.mark.parametrize("nbytes", [2 * CHUNK - 4, 2 * CHUNK, 2 * CHUNK + 4, 2 * CHUNK + 2, 1 << 20, RING - 4, RING, RING + 4,
+@pytest.mark.parametrize("nbytes", [2 * CHUNK - 4, 2 * CHUNK, 2 * CHUNK + 4, 2 * CHUNK + 2, 1 << 20,
+                                    8 * CHUNK - 4, 8 * CHUNK, 8 * CHUNK + 4, 8 * CHUNK + 2, 9 * CHUNK, RING - 4, RING, RING + 4,
                                     RING + CHUNK + 16, 3 * RING + 12, 13 << 20])
 @pytest.mark.parametrize("offset", [0, 4, 16])
 def test_lengths(A, nbytes, offset):

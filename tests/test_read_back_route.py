@@ -48,7 +48,9 @@ CASES = {
 lib.dh_init(0)
 for mb in (4, 13, 4, 9):
     expect(read(memory(mb * MB + 12)), "ring")
-expect(read(memory(1024)), "runtime")
+for nbytes in (1024, 512 << 10, MB, 2 * MB - 4):
+    expect(read(memory(nbytes)), "runtime")       # what gains nothing by the ring
+expect(read(memory(2 * MB)), "ring")
 """,
     "library on the second device": """
 lib.dh_init(1)
