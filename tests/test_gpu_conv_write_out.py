@@ -213,3 +213,39 @@ def test_small_paired_launches(A, shape):
             lib.dh_debug_force_splitk(0)
         for g, w, m, n in zip((y[i].cpu().numpy(), dx[i].cpu().numpy()), whole, mag, (kh * kw * C, kh * kw * O)):
             assert np.abs(g - w).max() <= 2.0 ** -24 * n * m.max()
+
+
+@pytest.mark.parametrize("generic", [0, 1])
+@pytest.mark.parametrize("splits", [0, 1, 2])
+@pytest.mark.parametrize("shape", [(2, 6, 6, 16, 3, 3, 16, 1), (2, 6, 6, 32, 3, 3, 70, 1), (2, 6, 6, 32, 3, 3, 132, 1)])
+def test_negative_zeros(A, shape, splits, generic):
+    """Sums of products that all underflow from below are -0, and stay that without a bias, with the activations that keep it; in
+    which launch they are formed makes no difference."""
+    print("shape", shape, "splits", splits, "generic", generic, flush=True)
+    be = A.HipBackend(0)
+    N, H, W, C, kh, kw, O, s = shape
+    x, k = np.full((N, H, W, C), 1e-30, np.float32), np.full((kh, kw, C, O), -1e-30, np.float32)
+    be.lib.dh_debug_force_splitk(splits)
+    be.lib.dh_debug_force_generic_conv(generic)
+    try:
+        for act in (A.ACT_NONE, A.ACT_RELU, A.ACT_LEAKY):
+            y = be.conv2d(x, k, (s, s), act=act, alpha=0.2)
+            inner = y[:, 1:-1, 1:-1]     # no tap in the padding, whose products are 0
+            assert (inner == 0).all() and np.signbit(inner).all(), act
+    finally:
+        be.lib.dh_debug_force_splitk(0)
+        be.lib.dh_debug_force_generic_conv(0)
+
+
+@pytest.mark.parametrize("shape", [(9, 27, 19, 48, 3, 3, 80, 1), (16, 9, 9, 128, 9, 9, 32, 1)])
+def test_negative_zeros_of_filter_gradients(A, shape):
+    """The same in whole filter gradients (in a split one the slices' own zeros may have either sign)."""
+    be = A.HipBackend(0)
+    N, H, W, C, kh, kw, O, s = shape
+    pads = (A.same_pad(H, kh, s)[0], A.same_pad(W, kw, s)[0])
+    be.lib.dh_debug_force_splitk(1)
+    try:
+        d = be.conv2d_kernel_grad(np.full((N, H, W, O), -1e-30, np.float32), np.full((N, H, W, C), 1e-30, np.float32), s, pads)
+    finally:
+        be.lib.dh_debug_force_splitk(0)
+    assert (d == 0).all() and np.signbit(d).all()
