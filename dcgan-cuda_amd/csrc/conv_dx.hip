@@ -86,7 +86,7 @@ int conv_dx(const char* who, const float* dy, const float* dy2, const float* k, 
             tiles += t;
             slabs += t * ((all[q].K + BK - 1) / BK);
         }
-        cfg = narrower_if_split(cfg, C, tiles, slabs);
+        cfg = narrower_if_split(cfg, C, tiles, slabs, [&] { return planned_in_two_groups<MODE_DX>(p, all, n_live, pair, tiles); });
         if (g_force_tile_width && cfg.bm == 128 && C > 64) cfg.bn = g_force_tile_width;
         if (g_tuning_width && cfg.bm == 128 && C > 64) cfg.bn = g_tuning_width;
         if (width_is_measured(cfg, tiles))

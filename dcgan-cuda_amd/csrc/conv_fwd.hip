@@ -45,7 +45,8 @@ int conv_fwd(const char* who, const float* x, const float* x2, const float* k, f
     if (takes_fast_path(veca, vecb))
     {
         const long tiles = (long)((p.phase[0].M + cfg.bm - 1) / cfg.bm) * ((O + cfg.bn - 1) / cfg.bn) * instances;
-        cfg = narrower_if_split(cfg, O, tiles, tiles * ((p.phase[0].K + BK - 1) / BK));
+        cfg = narrower_if_split(cfg, O, tiles, tiles * ((p.phase[0].K + BK - 1) / BK),
+                                [&] { return planned_in_two_groups<MODE_FWD>(p, p.phase, 1, pair, tiles); });
         if (g_force_tile_width && cfg.bm == 128 && O > 64) cfg.bn = g_force_tile_width;
         if (g_tuning_width && cfg.bm == 128 && O > 64) cfg.bn = g_tuning_width;
         if (width_is_measured(cfg, tiles))

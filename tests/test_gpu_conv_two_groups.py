@@ -1,0 +1,106 @@
+"""Launches whose workgroups are two groups of four wavefronts, each with half of the workgroup's k-slabs: shares that are odd or shorter
+than the rest, whole and split, remainders of rows and columns, batches that are and are not a multiple of 16, two operand pairs, an infinity in
+one group's slabs."""
+import os
+import shutil
+import subprocess
+
+import numpy as np
+import pytest
+
+from common import rand_conv_inputs, same_pad
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+
+# product, instances, (N, H, W, C, kh, kw, O, stride), cut: workgroups' share of slabs and slices of the longest tile
+CASES = [
+    ("fwd", 1, (37, 27, 19, 48, 3, 3, 80, 1), (27, 1)),      # whole, 27 slabs: 14 and 13; 37 images, 80 of 128 columns
+    ("fwd", 1, (16, 24, 20, 80, 3, 3, 132, 1), (23, 2)),     # two slices, the second a slab less; 4 columns in the second tile
+    ("fwd", 2, (16, 15, 13, 64, 5, 5, 128, 1), (20, 5)),     # pair
+    ("dx", 1, (40, 13, 12, 132, 3, 3, 112, 1), (32, 2)),     # remainder of rows, image-major
+    ("dx", 2, (32, 9, 9, 128, 3, 3, 160, 1), (15, 6)),       # pair
+    ("dk", 1, (6, 33, 31, 20, 5, 5, 68, 1), (8, 48)),        # smallest share, any batch, many slices shared by threads
+    ("dk", 1, (16, 19, 17, 20, 5, 5, 68, 1), (8, 41)),       # a slab is 16 images of one pixel
+    ("dk", 2, (16, 19, 17, 20, 5, 5, 132, 1), (20, 33)),     # two pairs of operands
+    ("dk", 1, (7, 40, 40, 32, 3, 3, 96, 1), (9, 78)),
+]
+
+
+@pytest.mark.parametrize("case", CASES)
+def test_cut_into_two_groups(case, tmp_path_factory):
+    """The launches below are the ones this file is about, and no unit gets two workgroups."""
+    hipcc = shutil.which("hipcc") or "/opt/rocm/bin/hipcc"
+    if not os.path.exists(hipcc):
+        pytest.skip("hipcc not found")
+    exe = str(tmp_path_factory.getbasetemp() / "two_groups_plan")
+    if not os.path.exists(exe):
+        subprocess.run([hipcc, "--cuda-host-only", "-O1", "-std=c++17", "-Wno-unused-function", "-I" + os.path.join(ROOT, "include"),
+                        "-I" + os.path.join(ROOT, "dcgan-cuda_amd", "csrc"), "-o", exe, os.path.join(ROOT, "tests", "two_groups_plan.hip")], check=True)
+    what, instances, (N, H, W, C, kh, kw, O, s), cut = case
+    out = subprocess.run([exe, what] + [str(v) for v in (N, H, W, C, O, kh, s, instances)], capture_output=True, text=True, check=True).stdout
+    groups, per, slices, workgroups = map(int, out.split())
+    assert (groups, (per, slices)) == (2, cut) and workgroups <= 256, out
+
+
+def products(be, what, x, x2, k, dy, dy2, shape, instances):
+    N, H, W, C, kh, kw, O, s = shape
+    pads = (same_pad(H, kh, s)[0], same_pad(W, kw, s)[0])
+    if what == "fwd":
+        return be.conv2d_pair(x, x2, k, (s, s)) if instances == 2 else (be.conv2d(x, k, (s, s)),)
+    if what == "dx":
+        return be.conv2d_input_grad_pair(dy, dy2, k, s, (H, W)) if instances == 2 else (be.conv2d_input_grad(dy, k, s, (H, W)),)
+    return (be.conv2d_kernel_grad_pair(dy, x, dy2, x2, s, pads) if instances == 2 else be.conv2d_kernel_grad(dy, x, s, pads),)
+
+
+def exact(orc64, what, x, x2, k, dy, dy2, shape, instances):
+    N, H, W, C, kh, kw, O, s = shape
+    pads = (same_pad(H, kh, s)[0], same_pad(W, kw, s)[0])
+    one = {"fwd": lambda a, g: orc64.conv2d(a, k, (s, s)), "dx": lambda a, g: orc64.conv2d_input_grad(g, k, s, (H, W)),
+           "dk": lambda a, g: orc64.conv2d_kernel_grad(g, a, s, pads)}[what]
+    both = [one(x, dy)] + ([one(x2, dy2)] if instances == 2 else [])
+    return (both[0] + both[-1],) if what == "dk" and instances == 2 else tuple(both)
+
+
+@pytest.fixture(scope="module")
+def be():
+    import __graft_entry__ as ge
+    return ge.load_package().HipBackend(0)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("case", CASES)
+def test_sums_of_both_groups(be, orc64, case):
+    """Against 64-bit sums.  A sum is rounded once per slab of 16 products in either of its two parts and once per slice, by 2^-23 of the
+    magnitudes added up at most (the matrix cores may cut off); the products themselves are good for 2^-24.  A slab that is missing or counted
+    twice is some hundred times that."""
+    what, instances, shape, _ = case
+    print("case", case, flush=True)
+    N, H, W, C, kh, kw, O, s = shape
+    x, k, dy = rand_conv_inputs(51, *shape)
+    x2, _, dy2 = rand_conv_inputs(52, *shape)
+    orc64.set_threads(8)
+    got = products(be, what, x, x2, k, dy, dy2, shape, instances)
+    again = products(be, what, x, x2, k, dy, dy2, shape, instances)
+    want = exact(orc64, what, x, x2, k, dy, dy2, shape, instances)
+    size = exact(orc64, what, *(np.abs(t) for t in (x, x2, k, dy, dy2)), shape, instances)
+    contraction = {"fwd": kh * kw * C, "dx": kh * kw * O, "dk": N * H * W * instances}[what]
+    for g, a, w, m in zip(got, again, want, size):
+        np.testing.assert_array_equal(g, a)
+        assert (np.abs(g - w) <= (contraction / 16 + 4) * 2.0 ** -23 * m).all(), np.max(np.abs(g - w) / m)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("tap", [(0, 0), (2, 2)])   # in the first group's slabs, in the second's
+def test_infinity_in_one_groups_slabs(be, orc, tap):
+    """One filter element is infinite: the infinities of its column are those of plain fp32 arithmetic; the other columns keep their values,
+    from either kind of products."""
+    shape = CASES[0][2]
+    x, k, dy = rand_conv_inputs(53, *shape)
+    plain = be.conv2d(x, k, (1, 1))
+    k[tap[0], tap[1], 5, 33] = np.inf
+    orc.set_threads(8)
+    got, want = be.conv2d(x, k, (1, 1)), orc.conv2d(x, k, (1, 1))
+    others = np.arange(shape[6]) != 33
+    np.testing.assert_array_equal(np.isposinf(got[..., 33]), np.isposinf(want[..., 33]))
+    np.testing.assert_array_equal(np.isneginf(got[..., 33]), np.isneginf(want[..., 33]))
+    np.testing.assert_allclose(got[..., others], plain[..., others], rtol=0, atol=2.0 ** -23 * 31 * 432 * 0.02)
