@@ -101,6 +101,9 @@ int conv_dx(const char* who, const float* dy, const float* dy2, const float* k, 
     }
     for (int q = 0; q < n_live; ++q)
         total_tiles_m += (all[q].M + cfg.bm - 1) / cfg.bm;
+    if (takes_fast_path(veca, vecb) && g_force_splitk == 0)
+        order_phases(all, n_live, cfg, (C + cfg.bn - 1) / cfg.bn * instances, total_tiles_m * ((C + cfg.bn - 1) / cfg.bn) * instances,
+                     TuneKey{MODE_DX, N, H, W, C, Ho, Wo, O, kh, kw, sh, sw, pad_top, pad_left, pair ? 1 : 0, num_cus()});
     if (takes_fast_path(veca, vecb))
     {
         p.skip = p.posmajor = skipping_pays(total_tiles_m * ((C + cfg.bn - 1) / cfg.bn) * instances);
