@@ -1,5 +1,5 @@
 // Filter-gradient entry points: dh_conv2d_dk, dh_conv2d_dk_pair (see conv_igemm.inc for the kernels).
-#include "conv_igemm.inc"
+#include "conv_tiny.inc"
 
 namespace
 {
@@ -45,6 +45,15 @@ int conv_dk(const char* who, const float* x, const float* dy, const float* x2, c
     g_operand_bytes = {(size_t)N * H * W * C * 4, (size_t)N * Ho * Wo * O * 4, true};
     if (pair && !takes_fast_path(veca, vecb))
         return fail(DH_ENOTSUP, "%s: the paired launch needs channel counts divisible by 4, 16-byte aligned tensors below 2 GiB", who);
+    if (!pair)
+    {
+        const TinyShape tiny = tiny_shape<MODE_DK>(p, p.phase, 1, takes_fast_path(veca, vecb));
+        if (tiny.tm)
+        {
+            g_prof_flops = 2.0 * N * Ho * Wo * O * kh * kw * C;
+            return launch_tiny<MODE_DK>(p, 1, p.phase[0].M, tiny, as_stream(stream));
+        }
+    }
     const long slabs_one = (p.phase[0].K + BK - 1) / BK;
     const TileCfg cfg = pick_tile(p.phase[0].M, O);
     if (takes_fast_path(veca, vecb))

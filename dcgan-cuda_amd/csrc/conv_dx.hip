@@ -1,6 +1,6 @@
 // Input-gradient / transposed-convolution entry points: dh_conv2d_dx, dh_conv2d_dx_pair (see
 // conv_igemm.inc for the kernels).
-#include "conv_igemm.inc"
+#include "conv_tiny.inc"
 
 #include <algorithm>
 
@@ -76,6 +76,17 @@ int conv_dx(const char* who, const float* dy, const float* dy2, const float* k, 
     if (pair && (!takes_fast_path(veca, vecb) || C % 4 != 0))
         return fail(DH_ENOTSUP, "%s: the paired launch needs dy channels divisible by 16, result channels divisible by 4, 16-byte aligned tensors below 2 GiB", who);
     const int instances = pair ? 2 : 1;
+    if (!pair)
+    {
+        const TinyShape tiny = tiny_shape<MODE_DX>(p, all, n_live, takes_fast_path(veca, vecb));
+        if (tiny.tm)
+        {
+            for (int q = 0; q < n_live; ++q)
+                p.phase[q] = all[q];
+            g_prof_flops = 2.0 * N * Ho * Wo * O * kh * kw * C;
+            return launch_tiny<MODE_DX>(p, n_live, max_m, tiny, as_stream(stream));
+        }
+    }
     TileCfg cfg = pick_tile(max_m, C);
     if (takes_fast_path(veca, vecb))
     {

@@ -1,5 +1,5 @@
 // Forward convolution entry points: dh_conv2d_fwd, dh_conv2d_fwd_pair (see conv_igemm.inc for the kernels).
-#include "conv_igemm.inc"
+#include "conv_tiny.inc"
 
 namespace
 {
@@ -40,6 +40,15 @@ int conv_fwd(const char* who, const float* x, const float* x2, const float* k, f
     g_operand_bytes = {(size_t)N * H * W * C * 4, (size_t)kh * kw * C * O * 4, C % BK == 0};
     if (pair && !takes_fast_path(veca, vecb))
         return fail(DH_ENOTSUP, "%s: the paired launch needs input channels divisible by 16, output channels divisible by 4, 16-byte aligned tensors below 2 GiB", who);
+    if (!pair)
+    {
+        const TinyShape tiny = tiny_shape<MODE_FWD>(p, p.phase, 1, takes_fast_path(veca, vecb));
+        if (tiny.tm)
+        {
+            g_prof_flops = 2.0 * N * Ho * Wo * O * kh * kw * C;
+            return launch_tiny<MODE_FWD>(p, 1, p.phase[0].M, tiny, as_stream(stream));
+        }
+    }
     TileCfg cfg = pick_tile(p.phase[0].M, O);
     const int instances = pair ? 2 : 1;
     if (takes_fast_path(veca, vecb))

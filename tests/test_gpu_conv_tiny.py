@@ -1,0 +1,108 @@
+"""Small launches, whose workgroups have an output tile of 16x16 to 32x32 each and share the contraction among their wavefronts: all four tiles, 16-byte
+and single loads, remainders of rows, columns and of the contraction, fewer steps than wavefronts, stride phases without a tap."""
+import numpy as np
+import pytest
+
+from common import rand_conv_inputs, same_pad
+
+pytestmark = pytest.mark.gpu
+
+# product, tile it must take, (N, H, W, C, kh, kw, O, stride)
+CASES = [
+    ("fwd", "16x16,8", (1, 16, 16, 128, 5, 5, 250, 2)),    # 100 steps, 16-byte loads of x, remainder of columns
+    ("fwd", "16x16,8", (1, 12, 13, 37, 3, 3, 29, 1)),      # 333 k: single loads, a lane's k in two taps
+    ("fwd", "32x16,8", (3, 27, 19, 48, 3, 3, 80, 1)),      # 14 steps for 8 wavefronts
+    ("fwd", "32x32,8", (20, 33, 33, 18, 4, 4, 30, 2)),
+    ("fwd", "32x32,4", (10, 40, 40, 10, 2, 2, 100, 2)),    # 40 k: two steps for four wavefronts
+    ("dx", "16x16,8", (1, 32, 32, 64, 5, 5, 128, 2)),      # phases of 9, 6, 6 and 4 taps
+    ("dx", "16x16,8", (8, 12, 13, 37, 3, 3, 29, 1)),
+    ("dx", "32x16,8", (2, 32, 32, 64, 5, 5, 128, 2)),
+    ("dx", "32x32,4", (4, 8, 9, 513, 1, 1, 96, 1)),        # one tap
+    ("dx", "32x32,4", (10, 21, 19, 40, 1, 1, 100, 2)),     # three of four phases have no tap: zeros
+    ("dk", "16x16,8", (1, 12, 13, 37, 3, 3, 29, 1)),
+    ("dk", "32x16,8", (4, 16, 16, 64, 5, 5, 64, 2)),
+    ("dk", "32x32,4", (1, 16, 16, 128, 5, 5, 256, 2)),     # two steps for four wavefronts
+    ("dk", "32x32,8", (2, 32, 32, 64, 5, 5, 128, 2)),
+]
+
+
+@pytest.fixture(scope="module")
+def A():
+    import __graft_entry__ as ge
+    return ge.load_package().hipabi
+
+
+@pytest.fixture(scope="module")
+def be(A):
+    return A.HipBackend(0)
+
+
+def product(be, what, x, k, dy, shape):
+    N, H, W, C, kh, kw, O, s = shape
+    if what == "fwd":
+        return be.conv2d(x, k, (s, s))
+    if what == "dx":
+        return be.conv2d_input_grad(dy, k, s, (H, W))
+    return be.conv2d_kernel_grad(dy, x, s, (same_pad(H, kh, s)[0], same_pad(W, kw, s)[0]))
+
+
+@pytest.mark.parametrize("case", CASES)
+def test_small_launches(A, be, orc64, case):
+    """Against 64-bit sums: a share of the contraction is rounded once per 16 products in either of its two parts, the shares of 8 wavefronts are added in either
+    part and the parts once, by 2^-23 of the magnitudes at most (the matrix cores may cut off); a step left out or counted twice is hundreds of times that."""
+    what, tile, shape = case
+    print("case", case, flush=True)
+    if A.device_info()["compute_units"] != 256:
+        pytest.skip("the tiles are those of a device with 256 compute units")
+    N, H, W, C, kh, kw, O, s = shape
+    x, k, dy = rand_conv_inputs(71, *shape)
+    A.profile_enable(1)
+    A.profile_reset()
+    try:
+        got = product(be, what, x, k, dy, shape)
+        tags = [r["name"] for r in A.profile_read()]
+    finally:
+        A.profile_enable(0)
+    assert tags == ["conv_tiny<%s,%s>" % (what, tile)]
+    np.testing.assert_array_equal(got, product(be, what, x, k, dy, shape))
+    orc64.set_threads(8)
+    want = product(orc64, what, x, k, dy, shape)
+    size = product(orc64, what, np.abs(x), np.abs(k), np.abs(dy), shape)
+    contraction = {"fwd": kh * kw * C, "dx": kh * kw * O, "dk": N * H * W}[what]
+    bound = (contraction / 8 / 16 + 12) * 2.0 ** -23 * size
+    assert (np.abs(got - want) <= bound).all(), np.max(np.abs(got - want) / np.maximum(bound, 1e-300))
+
+
+@pytest.mark.parametrize("act", ["none", "leaky", "tanh"])
+@pytest.mark.parametrize("what", ["fwd", "dx"])
+def test_bias_and_activation(A, be, what, act):
+    """(product + bias) through the activation, as from the product alone."""
+    shape = (2, 9, 7, 19, 3, 3, 21, 1)
+    N, H, W, C, kh, kw, O, s = shape
+    x, k, dy = rand_conv_inputs(72, *shape)
+    bias = np.random.default_rng(73).standard_normal(O if what == "fwd" else C).astype(np.float32)
+    kind = {"none": A.ACT_NONE, "leaky": A.ACT_LEAKY, "tanh": A.ACT_TANH}[act]
+    z = product(be, what, x, k, dy, shape) + bias
+    want = {"none": z, "leaky": np.where(z < 0, np.float32(0.2) * z, z), "tanh": np.tanh(z)}[act]
+    got = be.conv2d(x, k, (s, s), bias=bias, act=kind, alpha=0.2) if what == "fwd" else be.conv2d_input_grad(dy, k, s, (H, W), bias=bias, act=kind, alpha=0.2)
+    np.testing.assert_allclose(got, want, rtol=0 if act != "tanh" else 1e-6, atol=0 if act != "tanh" else 1e-7)
+
+
+@pytest.mark.parametrize("what", ["fwd", "dx", "dk"])
+@pytest.mark.parametrize("odd", ["infinity", "large", "many large"])
+def test_sums_that_parts_overflow_on(be, orc, what, odd):
+    """An infinity; products that bf16 parts overflow on (2^80 and more) in one wavefront's share; in all of them, where each share is below that and their sum is not."""
+    shape = (2, 6, 7, 32, 3, 3, 24, 1)
+    N, H, W, C, kh, kw, O, s = shape
+    x, k, dy = (np.abs(t) + np.float32(0.5) for t in rand_conv_inputs(74, *shape))
+    if odd == "infinity":
+        x[1, 2, 3, 4] = k[1, 1, 4, 5] = dy[1, 2, 3, 5] = np.inf
+    elif odd == "large":
+        x[1, 2, 3, 4] = k[1, 1, 4, 5] = dy[1, 2, 3, 5] = 2.0 ** 60
+    else:
+        x, k, dy = (t * np.float32(2.0 ** 37) for t in (x, k, dy))
+    orc.set_threads(8)
+    got, want = product(be, what, x, k, dy, shape), product(orc, what, x, k, dy, shape)
+    np.testing.assert_array_equal(np.isfinite(got), np.isfinite(want))
+    fine = np.isfinite(want)
+    np.testing.assert_allclose(got[fine], want[fine], rtol=288 * 2.0 ** -23, atol=0)     # all terms positive: 288 roundings at most
