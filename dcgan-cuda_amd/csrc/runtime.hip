@@ -2,6 +2,7 @@
 // Stands in for the GPU branches of the reference's src/memory (alloc.cu, copy.hxx).
 #include "dh_common.h"
 
+#include <algorithm>
 #include <atomic>
 #include <condition_variable>
 #include <cstdarg>
@@ -21,9 +22,11 @@ thread_local char g_err[512] = "";
 // the runtime where the current device keeps its copy and stores that pointer in the device state.
 __attribute__((used)) static __device__ __align__(256) unsigned char scratch[STATIC_SCRATCH_BYTES];
 
-// Chunks of a large copy to the host, see dh_memcpy_d2h.
-constexpr size_t READ_CHUNK = 256 * 1024;
-constexpr int READ_SLOTS = 16;
+// A large copy to the host, see dh_memcpy_d2h: it goes through a ring in pieces, and an event is recorded for up to four of them.
+constexpr size_t READ_PIECE = 256 * 1024;
+constexpr size_t READ_CHUNK_MAX = 4 * READ_PIECE;
+constexpr size_t READ_RING = 8 * READ_CHUNK_MAX;
+constexpr int READ_SLOTS_MAX = READ_RING / READ_PIECE;
 constexpr size_t READ_STAGED_MIN = 2 * 1024 * 1024;   // smaller ones gain nothing
 constexpr int READ_THREADS_MAX = 3;
 
@@ -41,9 +44,9 @@ struct DeviceState
     struct Stage { void* host; size_t bytes; hipEvent_t done; bool in_flight; };
     Stage stage[STAGE_SLOTS] = {};
     int next_stage = 0;
-    // pinned ring of dh_memcpy_d2h (READ_SLOTS chunks) and one event per chunk in flight; g_read_mu guards it
+    // pinned ring of dh_memcpy_d2h and one event per chunk in flight; g_read_mu guards it
     void* read_ring = nullptr;
-    hipEvent_t read_done[READ_SLOTS] = {};
+    hipEvent_t read_done[READ_SLOTS_MAX] = {};
     void* static_scratch = nullptr;   // this device's copy of `scratch`
 };
 
@@ -207,28 +210,48 @@ bool inside_memory_of(int device, const void* ptr, size_t bytes)
 
 constexpr int READ_NOT_STARTED = -1000;   // nothing was queued: the caller copies in another way
 
-// The chunks of a copy, shared by the thread that queues them and its helpers.  Chunk c goes through slot c % READ_SLOTS;
-// a slot is filled again only once the chunk before has been taken out of it.
+// A copy, shared by the thread that queues it and the helpers that take it out of the ring.  Both go by pieces, a launch each; a chunk is the
+// pieces of one event.  Chunk c goes through slot c % slots; a slot is filled again only once every piece of the chunk before has been taken.
+// Only the last chunk and the last piece are short, and nothing follows that chunk.
+// Queueing, recording and waiting for a piece of 256 KiB by itself takes the queueing thread 11 us, the bus 5: an event for four of them, or
+// for two where a copy has few, so that the first ones are there early.  Reading the weights of a model (38 MB in 18 calls) / sampling 64 images
+// (3.1 MB), us: an event per piece 1750 / 321, as here 1510 / 300.  Pieces of 128 KiB and more than three helpers: 0 to 12 % slower.
 struct Read
 {
     char* dst;
     const char* ring;
-    size_t bytes;
-    int chunks;
-    std::atomic<int> arrived{0};                    // chunks 0 ... arrived - 1 are in the ring
-    std::atomic<int> next{0};                       // next chunk to take out
-    std::atomic<bool> stop{false};                  // after an error: no further chunk will arrive
-    std::atomic<int> taken[READ_SLOTS] = {};        // chunks taken out of the slot so far
+    size_t bytes, chunk = READ_PIECE;
+    int chunks, slots, pieces, per_chunk;
+    std::atomic<int> arrived{0};                    // pieces 0 ... arrived - 1 are in the ring
+    std::atomic<int> next{0};                       // next piece to take out
+    std::atomic<bool> stop{false};                  // after an error: nothing further will arrive
+    std::atomic<int> taken[READ_SLOTS_MAX] = {};    // pieces taken out of the slot so far
     std::mutex mu;                                  // with `moved`: helpers sleep until the first chunk is there, however long the
     std::condition_variable moved;                  // work in front of the copy takes; the chunks after it are microseconds apart
 
-    size_t begin(int c) const { return (size_t)c * READ_CHUNK; }
-    size_t size(int c) const { return begin(c) + READ_CHUNK <= bytes ? READ_CHUNK : bytes - begin(c); }
-
-    void take(int c)
+    Read(char* to, const void* through, size_t n) : dst(to), ring(static_cast<const char*>(through)), bytes(n)
     {
-        memcpy(dst + begin(c), ring + (size_t)(c % READ_SLOTS) * READ_CHUNK, size(c));
-        taken[c % READ_SLOTS].fetch_add(1, std::memory_order_release);
+        while (chunk < READ_CHUNK_MAX && chunk < bytes / 6)
+            chunk *= 2;
+        slots = (int)(READ_RING / chunk);
+        per_chunk = (int)(chunk / READ_PIECE);
+        chunks = (int)((bytes + chunk - 1) / chunk);
+        pieces = (int)((bytes + READ_PIECE - 1) / READ_PIECE);
+    }
+    size_t begin(int c) const { return (size_t)c * chunk; }
+    size_t size(int c) const { return begin(c) + chunk <= bytes ? chunk : bytes - begin(c); }
+    int pieces_up_to(int c) const { return c + 1 < chunks ? (c + 1) * per_chunk : pieces; }
+    bool empty(int c) const     // the slot of chunk c, of the chunks before it
+    {
+        return taken[c % slots].load(std::memory_order_acquire) >= c / slots * per_chunk;
+    }
+
+    void take(int p)
+    {
+        const size_t from = (size_t)p * READ_PIECE;
+        const int slot = p / per_chunk % slots;
+        memcpy(dst + from, ring + (size_t)slot * chunk + (size_t)(p % per_chunk) * READ_PIECE, from + READ_PIECE <= bytes ? READ_PIECE : bytes - from);
+        taken[slot].fetch_add(1, std::memory_order_release);
     }
     template <class T>
     void announce(std::atomic<T>& what, T value)
@@ -245,15 +268,15 @@ struct Read
             std::unique_lock<std::mutex> lock(mu);
             moved.wait(lock, [this] { return arrived.load() > 0 || stop.load(); });
         }
-        for (int c = next.fetch_add(1); c < chunks; c = next.fetch_add(1))
+        for (int p = next.fetch_add(1); p < pieces; p = next.fetch_add(1))
         {
-            while (arrived.load(std::memory_order_acquire) <= c)
+            while (arrived.load(std::memory_order_acquire) <= p)
             {
                 if (stop.load(std::memory_order_acquire))
                     return;
                 std::this_thread::yield();
             }
-            take(c);
+            take(p);
         }
     }
 };
@@ -263,7 +286,7 @@ int read_staged(DeviceState& st, char* dst, const char* src, size_t bytes)
     if (!st.read_ring)
     {
         void* ring = nullptr;
-        if (hipHostMalloc(&ring, READ_CHUNK * READ_SLOTS, hipHostMallocDefault) != hipSuccess)
+        if (hipHostMalloc(&ring, READ_RING, hipHostMallocDefault) != hipSuccess)
         {
             (void)hipGetLastError();
             return READ_NOT_STARTED;
@@ -277,22 +300,24 @@ int read_staged(DeviceState& st, char* dst, const char* src, size_t bytes)
             }
         st.read_ring = ring;
     }
-    Read r;
-    r.dst = dst;
-    r.ring = static_cast<const char*>(st.read_ring);
-    r.bytes = bytes;
-    r.chunks = (int)((bytes + READ_CHUNK - 1) / READ_CHUNK);
+    Read r(dst, st.read_ring, bytes);
 
     // on the null stream, as the blocking copy: behind what it and the streams that synchronise with it hold
     auto queue = [&](int c) -> hipError_t {
-        hipLaunchKernelGGL(copy_from_pinned, dim3((unsigned)(r.size(c) / 4096 + 1)), dim3(256), 0, nullptr,
-                           static_cast<char*>(st.read_ring) + (size_t)(c % READ_SLOTS) * READ_CHUNK, src + r.begin(c), r.size(c), true);
-        const hipError_t launched = hipGetLastError();
-        return launched != hipSuccess ? launched : hipEventRecord(st.read_done[c % READ_SLOTS], nullptr);
+        for (size_t at = 0; at < r.size(c); at += READ_PIECE)
+        {
+            const size_t n = std::min(READ_PIECE, r.size(c) - at);
+            hipLaunchKernelGGL(copy_from_pinned, dim3((unsigned)(n / 4096 + 1)), dim3(256), 0, nullptr,
+                               static_cast<char*>(st.read_ring) + (size_t)(c % r.slots) * r.chunk + at, src + r.begin(c) + at, n, true);
+            const hipError_t launched = hipGetLastError();
+            if (launched != hipSuccess)
+                return launched;
+        }
+        return hipEventRecord(st.read_done[c % r.slots], nullptr);
     };
     hipError_t err = hipSuccess;
     int queued = 0;
-    for (; queued < r.chunks && queued < READ_SLOTS && err == hipSuccess; ++queued)
+    for (; queued < r.chunks && queued < r.slots && err == hipSuccess; ++queued)
         err = queue(queued);
 
     std::thread helper[READ_THREADS_MAX];
@@ -311,20 +336,20 @@ int read_staged(DeviceState& st, char* dst, const char* src, size_t bytes)
     }
     for (int c = 0; c < r.chunks && err == hipSuccess; ++c)
     {
-        err = hipEventSynchronize(st.read_done[c % READ_SLOTS]);
+        err = hipEventSynchronize(st.read_done[c % r.slots]);
         if (err != hipSuccess)
             break;
         if (helpers == 0)
-            r.take(c);
+            for (int p = c * r.per_chunk; p < r.pieces_up_to(c); ++p)
+                r.take(p);
         else if (c == 0)
-            r.announce(r.arrived, 1);
+            r.announce(r.arrived, r.pieces_up_to(0));
         else
-            r.arrived.store(c + 1, std::memory_order_release);
+            r.arrived.store(r.pieces_up_to(c), std::memory_order_release);
         // refill the slots that have been emptied; with all others in flight, wait for the oldest
         while (queued < r.chunks && err == hipSuccess)
         {
-            const bool empty = r.taken[queued % READ_SLOTS].load(std::memory_order_acquire) > queued / READ_SLOTS - 1;
-            if (empty)
+            if (r.empty(queued))
                 err = queue(queued++);
             else if (queued - (c + 1) > 0)
                 break;          // chunks are still under way: on to the next of them
@@ -332,6 +357,8 @@ int read_staged(DeviceState& st, char* dst, const char* src, size_t bytes)
                 std::this_thread::yield();
         }
     }
+    if (err == hipSuccess && helpers > 0)
+        r.help();                               // everything is there: what is left is shared
     if (err != hipSuccess)
     {
         (void)hipStreamSynchronize(nullptr);    // no copy into the ring outlives the call
@@ -454,12 +481,12 @@ int dh_memcpy_d2h(void* dst, const void* src, size_t bytes)
 {
     DH_TRY(ensure_init());
     if (bytes == 0) return 0;
-    // Large copies go through a pinned ring (4 MiB a device, kept), a chunk at a time: the device fills the next slots while
+    // Large copies go through a pinned ring (8 MiB a device, kept), a chunk at a time: the device fills the next slots while
     // the host empties the ones that are there, with helper threads, since the page faults and the copy of one thread are
     // slower than the bus.  The runtime's own copy into pageable memory takes turns: a chunk across the bus, a wait, its copy.
-    // Measured: a stretch of six training iterations at batch 64 that ends with reading all weights (38 MB in 18 pieces) 20.5 -> 17.9 ms,
+    // Measured: a stretch of six training iterations at batch 64 that ends with reading all weights (38 MB in 18 calls) 20.5 -> 17.9 ms,
     // sampling 64 images (3.1 MB) 445 -> 395 us.  From 2 MiB on, where two helpers pay: runtime / ring, us, 2 MiB 119 / 98, 4 MiB 230 / 176,
-    // 13 MiB 717 / 505.  With one helper, which does all the copying while the caller waits, or with none the ring gained nothing: 512 KiB
+    // 13 MiB 717 / 505 (with an event for every 256 KiB; see struct Read for what several to an event give).  With one helper, which does all the copying while the caller waits, or with none the ring gained nothing: 512 KiB
     // 29.9 / 31.9, 1 MiB 58 / 61, 1.75 MiB 102 / 103 (medians).
     // Small ones, a copy while another is in progress, host memory that the device reaches by itself (pinned, managed) and
     // whatever is not inside one allocation on the library's device, that being the thread's too, take the runtime's copy, which finds

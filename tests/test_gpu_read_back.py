@@ -39,6 +39,15 @@ def test_lengths(A, nbytes, offset):
         np.testing.assert_array_equal(read(A, a.data_ptr() + offset, nbytes), exp[offset:offset + nbytes])
 
 
+@pytest.mark.parametrize("nbytes", [(3 << 20) - 4, 3 << 20, (3 << 20) + 4, (6 << 20) + CHUNK, (8 << 20) - 4, 8 << 20, (8 << 20) + 4,
+                                    (9 << 20) + 3 * CHUNK + 8, 17 << 20, (24 << 20) + 2 * CHUNK - 4])
+def test_lengths_around_the_pieces_of_an_event(A, nbytes):
+    """Two or four pieces to an event, slots that are filled again, a last chunk of fewer pieces."""
+    print("bytes", nbytes, flush=True)
+    a = torch.randint(0, 256, (nbytes,), dtype=torch.uint8, device="cuda")
+    np.testing.assert_array_equal(read(A, a.data_ptr(), nbytes), a.cpu().numpy())
+
+
 def test_behind_queued_work(A):
     a = torch.zeros(3 << 20, device="cuda")
     for i in range(5):
