@@ -1,0 +1,74 @@
+"""Results whose columns are no multiple of 4: the write-out turns 32 x 32 tiles in LDS.  Around the widths where that begins, the tiles' edges and
+remainders, direct and from slices, with and without a result that starts at 16 bytes; nothing outside the result is written."""
+import numpy as np
+import pytest
+import torch
+
+from common import ATOL, RTOL, rand_conv_inputs, same_pad
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def A():
+    import __graft_entry__ as ge
+    A = ge.load_package().hipabi
+    A.check(A.load().dh_init(0))
+    return A
+
+
+def guarded(shape, first):
+    """(whole buffer, pointer to its part that is the result): 64 words around it, which starts `first` words past 256 bytes."""
+    n = int(np.prod(shape))
+    whole = torch.full((n + 128,), 7.5, device="cuda")
+    return whole, whole.data_ptr() + 4 * (64 + first)
+
+
+def result(whole, shape, first):
+    torch.cuda.synchronize()
+    n, got = int(np.prod(shape)), whole.cpu().numpy()
+    assert (got[:64 + first] == 7.5).all() and (got[64 + first + n:] == 7.5).all()
+    return got[64 + first:64 + first + n].reshape(shape)
+
+
+@pytest.mark.parametrize("splits", [1, 3])
+@pytest.mark.parametrize("shape", [      # N, H, W, C, kh, kw, O, stride
+    (3, 9, 11, 16, 3, 3, 17, 1),         # the narrowest that is turned
+    (2, 10, 9, 18, 3, 3, 15, 1),         # columns one way are, the other way not
+    (3, 13, 7, 23, 3, 2, 31, 1),         # one tile, almost full
+    (2, 11, 12, 33, 3, 3, 34, 2),        # two columns in the second tile of 32
+    (3, 10, 10, 49, 2, 2, 50, 1),        # 18 in the second
+    (2, 17, 9, 65, 3, 3, 63, 1),
+    (5, 12, 13, 81, 3, 3, 98, 2),        # tiles of 128
+    (2, 15, 16, 127, 1, 1, 129, 1),      # and one column past one
+    (9, 30, 31, 37, 3, 3, 101, 1),       # many rows, the last tile a part
+    (4, 16, 16, 24, 3, 3, 40, 1),        # multiples of 4 at any address
+])
+@pytest.mark.parametrize("first", [0, 1])
+def test_write_out(A, orc, shape, splits, first):
+    print("shape", shape, "splits", splits, "first", first, flush=True)
+    N, H, W, C, kh, kw, O, s = shape
+    (ph, Ho), (pw, Wo) = A.same_pad(H, kh, s), A.same_pad(W, kw, s)
+    x, k, dy = rand_conv_inputs(71, *shape)
+    bias, bias_c = np.linspace(-0.5, 0.5, O).astype(np.float32), np.linspace(-0.3, 0.3, C).astype(np.float32)
+    orc.set_threads(8)
+    exp = (orc.relu_leaky(orc.bias_add(orc.conv2d(x, k, (s, s)), bias), 0.2),
+           orc.tanh(orc.bias_add(orc.conv2d_input_grad(dy, k, s, (H, W)), bias_c)),
+           orc.conv2d_kernel_grad(dy, x, s, (same_pad(H, kh, s)[0], same_pad(W, kw, s)[0])))
+    dx, dk, ddy, db, dbc = (torch.from_numpy(np.ascontiguousarray(a)).cuda() for a in (x, k, dy, bias, bias_c))
+    lib, p = A.load(), torch.Tensor.data_ptr
+    fwd = (N, H, W, C, kh, kw, O, s, s, ph // 2, pw // 2, Ho, Wo)
+    adj = (N, Ho, Wo, O, kh, kw, C, s, s, ph // 2, pw // 2, H, W)
+    fil = (N, H, W, C, Ho, Wo, O, kh, kw, s, s, ph // 2, pw // 2)
+    (wy, y), (wx, gx), (wk, gk) = (guarded(e.shape, first) for e in exp)
+    lib.dh_debug_force_splitk(splits)
+    try:
+        A.check(lib.dh_conv2d_fwd(p(dx), p(dk), y, *fwd, p(db), A.ACT_LEAKY, 0.2, None))
+        A.check(lib.dh_conv2d_dx(p(ddy), p(dk), gx, *adj, p(dbc), A.ACT_TANH, 0.0, None))
+        A.check(lib.dh_conv2d_dk(p(dx), p(ddy), gk, *fil, None))
+    finally:
+        lib.dh_debug_force_splitk(0)
+    for what, whole, e in zip(("fwd", "dx", "dk"), (wy, wx, wk), exp):
+        # sums of N*Ho*Wo products of U(-1,1) values: the filter gradient's absolute tolerance follows their magnitude
+        scale = max(1.0, float(np.abs(e).max())) if what == "dk" else 1.0
+        np.testing.assert_allclose(result(whole, e.shape, first), e, rtol=RTOL, atol=ATOL * scale, err_msg=what)
