@@ -72,3 +72,44 @@ def test_write_out(A, orc, shape, splits, first):
         # sums of N*Ho*Wo products of U(-1,1) values: the filter gradient's absolute tolerance follows their magnitude
         scale = max(1.0, float(np.abs(e).max())) if what == "dk" else 1.0
         np.testing.assert_allclose(result(whole, e.shape, first), e, rtol=RTOL, atol=ATOL * scale, err_msg=what)
+
+
+@pytest.mark.parametrize("shape", [      # N, H, W, C, kh, kw, O, stride
+    (40, 60, 61, 90, 1, 1, 1, 1),        # one column: chunks of four rows
+    (3, 21, 20, 91, 1, 1, 33, 1),        # the last chunk one element past the end
+    (3, 21, 20, 93, 3, 3, 66, 2),        # two
+    (3, 20, 21, 97, 2, 2, 103, 1),       # three
+    (1, 1, 1, 120, 1, 1, 3, 1),          # filter gradient over three elements
+    (1, 1, 2, 120, 1, 1, 1, 1),          # and over two
+    (1, 1, 1, 120, 1, 1, 5, 1),          # five
+])
+@pytest.mark.parametrize("first", [0, 1, 3])
+def test_rows_read_16_bytes_at_a_time(A, orc, shape, first):
+    """Filter and gradient that end and begin beside NaNs, at any address: nothing outside them gets into a result."""
+    print("shape", shape, "first", first, flush=True)
+    N, H, W, C, kh, kw, O, s = shape
+    (ph, Ho), (pw, Wo) = A.same_pad(H, kh, s), A.same_pad(W, kw, s)
+    x, k, dy = rand_conv_inputs(72, *shape)
+    orc.set_threads(8)
+    exp = orc.conv2d(x, k, (s, s)), orc.conv2d_kernel_grad(dy, x, s, (same_pad(H, kh, s)[0], same_pad(W, kw, s)[0]))
+
+    def among_nans(a):
+        whole = torch.full((a.size + 128,), float("nan"), device="cuda")
+        whole[64 + first:64 + first + a.size] = torch.from_numpy(np.ascontiguousarray(a).reshape(-1)).cuda()
+        return whole, whole.data_ptr() + 4 * (64 + first)
+
+    dx = torch.from_numpy(np.ascontiguousarray(x)).cuda()
+    (wf, f), (wd, d) = among_nans(k), among_nans(dy)
+    (wy, y), (wk, gk) = (guarded(e.shape, 0) for e in exp)
+    lib = A.load()
+    lib.dh_debug_force_splitk(1)
+    lib.dh_debug_force_generic_conv(1)
+    try:
+        A.check(lib.dh_conv2d_fwd(dx.data_ptr(), f, y, N, H, W, C, kh, kw, O, s, s, ph // 2, pw // 2, Ho, Wo, None, A.ACT_NONE, 0.0, None))
+        A.check(lib.dh_conv2d_dk(dx.data_ptr(), d, gk, N, H, W, C, Ho, Wo, O, kh, kw, s, s, ph // 2, pw // 2, None))
+    finally:
+        lib.dh_debug_force_generic_conv(0)
+        lib.dh_debug_force_splitk(0)
+    for what, whole, e in zip(("fwd", "dk"), (wy, wk), exp):
+        scale = max(1.0, float(np.abs(e).max())) if what == "dk" else 1.0
+        np.testing.assert_allclose(result(whole, e.shape, 0), e, rtol=RTOL, atol=ATOL * scale, err_msg=what)
