@@ -47,11 +47,12 @@ int conv_dk(const char* who, const float* x, const float* dy, const float* x2, c
         return fail(DH_ENOTSUP, "%s: the paired launch needs channel counts divisible by 4, 16-byte aligned tensors below 2 GiB", who);
     if (!pair)
     {
-        const TinyShape tiny = tiny_shape<MODE_DK>(p, p.phase, 1, takes_fast_path(veca, vecb));
+        const bool fast = takes_fast_path(veca, vecb);
+        const TinyShape tiny = tiny_shape<MODE_DK>(p, p.phase, 1, fast);
         if (tiny.tm)
         {
             g_prof_flops = 2.0 * N * Ho * Wo * O * kh * kw * C;
-            return launch_tiny<MODE_DK>(p, 1, p.phase[0].M, tiny, as_stream(stream));
+            return launch_tiny<MODE_DK>(p, 1, p.phase[0].M, tiny, fast, as_stream(stream));
         }
     }
     const long slabs_one = (p.phase[0].K + BK - 1) / BK;

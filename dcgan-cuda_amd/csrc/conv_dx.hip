@@ -78,13 +78,14 @@ int conv_dx(const char* who, const float* dy, const float* dy2, const float* k, 
     const int instances = pair ? 2 : 1;
     if (!pair)
     {
-        const TinyShape tiny = tiny_shape<MODE_DX>(p, all, n_live, takes_fast_path(veca, vecb));
+        const bool fast = takes_fast_path(veca, vecb);
+        const TinyShape tiny = tiny_shape<MODE_DX>(p, all, n_live, fast);
         if (tiny.tm)
         {
             for (int q = 0; q < n_live; ++q)
                 p.phase[q] = all[q];
             g_prof_flops = 2.0 * N * Ho * Wo * O * kh * kw * C;
-            return launch_tiny<MODE_DX>(p, n_live, max_m, tiny, as_stream(stream));
+            return launch_tiny<MODE_DX>(p, n_live, max_m, tiny, fast, as_stream(stream));
         }
     }
     TileCfg cfg = pick_tile(max_m, C);

@@ -42,11 +42,12 @@ int conv_fwd(const char* who, const float* x, const float* x2, const float* k, f
         return fail(DH_ENOTSUP, "%s: the paired launch needs input channels divisible by 16, output channels divisible by 4, 16-byte aligned tensors below 2 GiB", who);
     if (!pair)
     {
-        const TinyShape tiny = tiny_shape<MODE_FWD>(p, p.phase, 1, takes_fast_path(veca, vecb));
+        const bool fast = takes_fast_path(veca, vecb);
+        const TinyShape tiny = tiny_shape<MODE_FWD>(p, p.phase, 1, fast);
         if (tiny.tm)
         {
             g_prof_flops = 2.0 * N * Ho * Wo * O * kh * kw * C;
-            return launch_tiny<MODE_FWD>(p, 1, p.phase[0].M, tiny, as_stream(stream));
+            return launch_tiny<MODE_FWD>(p, 1, p.phase[0].M, tiny, fast, as_stream(stream));
         }
     }
     TileCfg cfg = pick_tile(p.phase[0].M, O);

@@ -4,6 +4,7 @@ import numpy as np
 import pytest
 
 from common import rand_conv_inputs, same_pad
+from test_gpu_conv_split_products import products64
 
 pytestmark = pytest.mark.gpu
 
@@ -106,3 +107,51 @@ def test_sums_that_parts_overflow_on(be, orc, what, odd):
     np.testing.assert_array_equal(np.isfinite(got), np.isfinite(want))
     fine = np.isfinite(want)
     np.testing.assert_allclose(got[fine], want[fine], rtol=288 * 2.0 ** -23, atol=0)     # all terms positive: 288 roundings at most
+
+
+GENERAL = [   # launches that the general kernel would take: channel counts that its wide loads or the buffer-load kernel do not fit
+    ("fwd", (1, 12, 13, 37, 3, 3, 29, 1)),
+    ("fwd", (20, 33, 33, 18, 4, 4, 30, 2)),
+    ("fwd", (10, 40, 40, 10, 2, 2, 100, 2)),
+    ("fwd", (2, 6, 6, 16, 3, 3, 17, 1)),      # 4.5 steps for 8 wavefronts, 16-byte loads
+    ("fwd", (1, 9, 9, 1, 1, 1, 5, 1)),        # one product per sum
+    ("dx", (8, 12, 13, 37, 3, 3, 29, 1)),
+    ("dx", (10, 21, 19, 40, 1, 1, 100, 2)),   # three of four phases have no tap
+    ("dx", (3, 9, 9, 5, 1, 1, 1, 1)),
+    ("dx", (2, 7, 7, 6, 3, 3, 24, 2)),        # 16-byte loads
+    ("dk", (1, 12, 13, 37, 3, 3, 29, 1)),
+    ("dk", (5, 3, 4, 7, 2, 2, 9, 1)),
+    ("dk", (1, 1, 1, 7, 1, 1, 9, 1)),
+]
+
+
+@pytest.mark.parametrize("case", GENERAL)
+def test_no_part_of_a_product_is_left_out(A, be, case):
+    """Where the general kernel would multiply in fp32.  At most one product of a sum is not zero here, and 32-bit arithmetic rounds it once.  Of nine products of bf16
+    parts the one of the high parts is exact; the others add up to 2^-7 of the product at most, of which the last two steps of that sum may cut off 2^-23 each and
+    the steps before them (at most 2^-15 of it) less: 2^-28.  (Six of the nine are 2^-27 off as a rule, 2^-24 at most.)"""
+    what, shape = case
+    print("case", case, flush=True)
+    N, H, W, C, kh, kw, O, s = shape
+    x, k, dy = rand_conv_inputs(75, *shape)
+    if what == "dk":
+        alone = np.zeros_like(x)        # one pixel of one image
+        alone[N // 2, H // 2, W // 2] = x[N // 2, H // 2, W // 2]
+        x = alone
+    else:
+        of = x if what == "fwd" else dy
+        step = (kh, kw) if what == "fwd" else (-(-kh // s), -(-kw // s))
+        alone = np.zeros_like(of)       # one channel of pixels so far apart that no result meets two
+        at = np.s_[:, ::step[0], ::step[1], of.shape[3] // 2]
+        alone[at] = of[at]
+        x, dy = (alone, dy) if what == "fwd" else (x, alone)
+    A.profile_enable(1)
+    A.profile_reset()
+    try:
+        got = product(be, what, x, k, dy, shape)
+        tags = [r["name"] for r in A.profile_read()]
+    finally:
+        A.profile_enable(0)
+    assert len(tags) == 1 and tags[0].startswith("conv_tiny<" + what)
+    exact = products64(x, k, dy, s)[what]
+    np.testing.assert_array_less(np.abs(got - exact), 0.5 * np.spacing(np.abs(got)) + 2.0 ** -28 * np.abs(exact) + 1e-300)
