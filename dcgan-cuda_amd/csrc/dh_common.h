@@ -82,8 +82,9 @@ int conv_dk_thin(const float* x, const float* dy, const float* x2, const float* 
 // Whether conv_dk_thin takes this geometry (16-byte aligned operands assumed).
 bool dk_thin_takes(int N, int H, int W, int C, int Ho, int Wo, int O, int kh, int kw, int sw);
 
-// Test and tuning switches (dh_debug_force_generic_conv, dh_debug_force_splitk).
+// Test and tuning switches (dh_debug_force_generic_conv, dh_debug_force_tiled_conv, dh_debug_force_splitk, dh_debug_force_tile_width).
 extern bool g_force_generic;  // route every convolution through the general kernel
+extern bool g_force_tiled;    // small launches too take the tiled kernels, cut as these choose
 extern int g_force_splitk;    // > 0: this many k splits (at most one per k-slab) instead of the automatic choice
 extern int g_force_tile_width;  // 64 / 128: width of the 128-row tiles of wide forward / input-gradient launches
 

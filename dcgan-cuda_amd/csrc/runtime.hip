@@ -168,6 +168,7 @@ int workspace(size_t bytes, void** ptr, hipStream_t stream)
 }
 
 bool g_force_generic = false;
+bool g_force_tiled = false;
 int g_force_splitk = 0;
 int g_force_tile_width = 0;
 
@@ -619,6 +620,12 @@ size_t dh_workspace_bytes(void)
 int dh_debug_force_generic_conv(int on)
 {
     g_force_generic = on != 0;
+    return 0;
+}
+
+int dh_debug_force_tiled_conv(int on)
+{
+    g_force_tiled = on != 0;
     return 0;
 }
 

@@ -46,6 +46,7 @@ _SIGS = {
     "dh_pool_trim": [],
     "dh_pool_stats": [C.POINTER(_sz)] * 4,
     "dh_debug_force_generic_conv": [_i],
+    "dh_debug_force_tiled_conv": [_i],
     "dh_debug_force_splitk": [_i],
     "dh_debug_force_tile_width": [_i],
     "dh_sigmoid_cross_entropy_head": [_vp] * 9 + [_sz, _vp],

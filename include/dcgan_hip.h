@@ -124,6 +124,10 @@ int dh_profile_read(char* buf, size_t buf_len);
  * checks, any channel count or alignment) even where the 16-byte buffer-load kernel applies. */
 int dh_debug_force_generic_conv(int on);
 
+/* Test hook: on != 0 keeps small single launches off the kernel that gives each workgroup an output tile of 16x16 to 32x32 to
+ * itself: they take the tiled kernels (buffer-load or general), cut along the contraction as these choose. */
+int dh_debug_force_tiled_conv(int on);
+
 /* Test and tuning hook: splits > 0 makes every convolution cut its contraction into that many
  * splits (at most one per 16-deep k-slab) instead of choosing by occupancy; 0 restores the choice.
  * The partial sums are added in split order by a second kernel, so results are reproducible. */

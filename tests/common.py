@@ -4,6 +4,8 @@
 operator tests -- through a backend `be` that offers the operator methods of `oracle.Oracle`
 (the HIP front-end offers the same ones) and returns the tensors the reference test exports.
 """
+import contextlib
+
 import numpy as np
 
 # north_star tolerance for fp32 results: 1e-4 relative / 1e-5 absolute
@@ -184,3 +186,21 @@ def rand_conv_inputs(seed, N, H, W, C, kh, kw, O, s):
     Ho, Wo = -(-H // s), -(-W // s)
     dy = rng.uniform(-1, 1, (N, Ho, Wo, O)).astype(np.float32)
     return x, k, dy
+
+
+@contextlib.contextmanager
+def convolutions(way, level=1):
+    """The convolution launches made inside, by the tags of the profiling interface: the list that is yielded holds them afterwards.  way: "tiled" keeps
+    small launches on the tiled kernels, anything else leaves the choice to the library.  level: 2 records every tagged kernel."""
+    import __graft_entry__ as ge
+    A = ge.load_package().hipabi
+    tags = []
+    A.check(A.load().dh_debug_force_tiled_conv(int(way == "tiled")))
+    A.profile_enable(level)
+    A.profile_reset()
+    try:
+        yield tags
+        tags += [r["name"] for r in A.profile_read()]
+    finally:
+        A.profile_enable(0)
+        A.check(A.load().dh_debug_force_tiled_conv(0))

@@ -5,7 +5,7 @@ reduction for the filter gradient whose sums run over the whole batch."""
 import numpy as np
 import pytest
 
-from common import RTOL, ATOL, rand_conv_inputs, same_pad
+from common import RTOL, ATOL, convolutions, rand_conv_inputs, same_pad
 
 pytestmark = pytest.mark.gpu
 
@@ -36,18 +36,29 @@ def close(got, exp, scale=1.0, what=""):
     np.testing.assert_allclose(got, exp, rtol=RTOL, atol=ATOL * scale, err_msg=what)
 
 
+def on_tiled_kernels(tags, shape):
+    """Whether launches that were kept on the tiled kernels ran there: the buffer-load one where both channel counts fit it, else that or the general
+    one, or the image layer's."""
+    fits = shape[3] % 16 == 0 and shape[6] % 16 == 0
+    return all(t.startswith("conv_igemm_fast<" if fits else ("conv_igemm", "fwd_", "dx_", "dk_")) for t in tags)
+
+
+@pytest.mark.parametrize("way", ["tiled", "small"])     # small: what the library chooses, for most of these conv_tiny
 @pytest.mark.parametrize("shape", SHAPES)
-def test_conv_fwd_dx_dk(be, orc, shape):
-    print("shape", shape, flush=True)
+def test_conv_fwd_dx_dk(be, orc, shape, way):
+    print("shape", shape, way, flush=True)
     N, H, W, C, kh, kw, O, s = shape
     x, k, dy = rand_conv_inputs(42, *shape)
     pads = (same_pad(H, kh, s)[0], same_pad(W, kw, s)[0])
     orc.set_threads(8)
-    close(be.conv2d(x, k, (s, s)), orc.conv2d(x, k, (s, s)), what="fwd")
-    close(be.conv2d_input_grad(dy, k, s, (H, W)), orc.conv2d_input_grad(dy, k, s, (H, W)), what="dx")
+    with convolutions(way) as tags:
+        y, dx, dk = be.conv2d(x, k, (s, s)), be.conv2d_input_grad(dy, k, s, (H, W)), be.conv2d_kernel_grad(dy, x, s, pads)
+    assert way == "small" or on_tiled_kernels(tags, shape), tags
+    close(y, orc.conv2d(x, k, (s, s)), what="fwd")
+    close(dx, orc.conv2d_input_grad(dy, k, s, (H, W)), what="dx")
     exp = orc.conv2d_kernel_grad(dy, x, s, pads)
     # sums of N*Ho*Wo products of U(-1,1) values: absolute tolerance follows their magnitude
-    close(be.conv2d_kernel_grad(dy, x, s, pads), exp, scale=max(1.0, float(np.abs(exp).max())), what="dk")
+    close(dk, exp, scale=max(1.0, float(np.abs(exp).max())), what="dk")
 
 
 @pytest.mark.parametrize("shape", [(2, 4, 4, 512, 5, 5, 256, 2), (2, 32, 32, 64, 5, 5, 3, 2), (3, 5, 7, 6, 3, 3, 4, 2)])
@@ -67,10 +78,11 @@ def test_conv_transpose_and_grads(be, orc, shape):
 
 
 @pytest.mark.parametrize("act", ["none", "relu", "leaky", "tanh", "sigmoid"])
+@pytest.mark.parametrize("way", ["tiled", "small"])
 @pytest.mark.parametrize("shape", [(2, 16, 16, 32, 5, 5, 64, 2), (4, 8, 8, 256, 5, 5, 512, 2), (1, 7, 9, 2, 3, 3, 5, 2)])
-def test_fused_epilogues(be, orc, act, shape):
+def test_fused_epilogues(be, orc, act, shape, way):
     """conv + bias + activation in one call == the three reference operators in sequence;
-    the second shape takes the split-K path, where the epilogue runs in the reduction."""
+    on the tiled kernels the first two shapes take the split-K path, where the epilogue runs in the reduction."""
     import __graft_entry__ as ge
     A = ge.load_package().hipabi
     N, H, W, C, kh, kw, O, s = shape
@@ -80,10 +92,15 @@ def test_fused_epilogues(be, orc, act, shape):
     f = {"none": lambda v: v, "relu": orc.relu, "leaky": lambda v: orc.relu_leaky(v, 0.2), "tanh": orc.tanh,
          "sigmoid": orc.sigmoid}[act]
     b = (rng.standard_normal(O) * 0.5).astype(np.float32)
-    close(be.conv2d(x, k, (s, s), bias=b, act=code, alpha=0.2), f(orc.bias_add(orc.conv2d(x, k, (s, s)), b)))
     bc = (rng.standard_normal(C) * 0.5).astype(np.float32)
-    close(be.conv2d_input_grad(dy, k, s, (H, W), bias=bc, act=code, alpha=0.2),
-          f(orc.bias_add(orc.conv2d_input_grad(dy, k, s, (H, W)), bc)))
+    with convolutions(way, level=2) as tags:
+        y = be.conv2d(x, k, (s, s), bias=b, act=code, alpha=0.2)
+        dx = be.conv2d_input_grad(dy, k, s, (H, W), bias=bc, act=code, alpha=0.2)
+    kernels = [t for t in tags if not t.startswith("hbm:")]
+    assert way == "small" or on_tiled_kernels(kernels, shape), tags
+    assert way == "small" or N == 1 or any("splitk_reduce" in t for t in tags), tags
+    close(y, f(orc.bias_add(orc.conv2d(x, k, (s, s)), b)))
+    close(dx, f(orc.bias_add(orc.conv2d_input_grad(dy, k, s, (H, W)), bc)))
 
 
 @pytest.mark.parametrize("shape", [(5, 12, 12, 36, 5, 5, 72, 2), (2, 32, 32, 64, 5, 5, 128, 2), (4, 8, 8, 256, 5, 5, 512, 2)])
@@ -338,12 +355,13 @@ def test_forced_split_counts(be, orc, shape, generic):
     (64, 16, 16, 16, 5, 5, 16, 2),   # ... 64 pixels per stride phase (the most the pixel table holds)
     (64, 6, 6, 16, 3, 3, 16, 1),     # ... stride 1
 ])
-@pytest.mark.parametrize("splits", [0, 5])
-def test_taps_in_the_padding_are_skipped(be, orc, shape, splits):
+@pytest.mark.parametrize("splits,way", [(0, "tiled"), (0, "small"), (5, "tiled")])
+def test_taps_in_the_padding_are_skipped(be, orc, shape, splits, way):
     """Shapes on which the buffer-load kernel leaves out the k-slabs whose taps fall into the
     padding (channel and image counts divisible by 16): forward, input gradient and filter gradient,
-    single and paired, automatic split and a forced one, against the oracle."""
-    padding_skip_case(be, orc, shape, splits)
+    single and paired, automatic split and a forced one, against the oracle; and the single launches as the
+    library chooses, which are small ones."""
+    padding_skip_case(be, orc, shape, splits, way)
 
 
 @pytest.mark.parametrize("seed", range(16))
@@ -353,13 +371,13 @@ def test_seeded_random_geometries_with_skipped_taps(be, orc, seed):
     kh, kw = int(rng.integers(2, 6)), int(rng.integers(2, 6))
     shape = (16 * int(rng.integers(1, 6)), int(rng.integers(1, 11)), int(rng.integers(1, 11)), 16 * int(rng.integers(1, 4)),
              kh, kw, 16 * int(rng.integers(1, 6)), int(rng.integers(1, 3)))
-    padding_skip_case(be, orc, shape, int(rng.integers(0, 7)))
+    padding_skip_case(be, orc, shape, int(rng.integers(0, 7)), "tiled")
 
 
-def padding_skip_case(be, orc, shape, splits):
+def padding_skip_case(be, orc, shape, splits, way):
     import __graft_entry__ as ge
     A = ge.load_package().hipabi
-    print("shape", shape, "splits", splits, flush=True)
+    print("shape", shape, "splits", splits, way, flush=True)
     N, H, W, C, kh, kw, O, s = shape
     x, k, dy = rand_conv_inputs(31, *shape)
     x2, _, dy2 = rand_conv_inputs(32, *shape)
@@ -371,10 +389,14 @@ def padding_skip_case(be, orc, shape, splits):
     exp_k = orc.conv2d_kernel_grad(dy, x, s, pads)
     be.lib.dh_debug_force_splitk(splits)
     try:
-        close(be.conv2d(x, k, (s, s), bias=bias, act=A.ACT_LEAKY, alpha=0.2), exp_f, what="fwd")
-        close(be.conv2d_input_grad(dy, k, s, (H, W)), exp_x, what="dx")
+        with convolutions(way) as tags:
+            y = be.conv2d(x, k, (s, s), bias=bias, act=A.ACT_LEAKY, alpha=0.2)
+            dx, dk = be.conv2d_input_grad(dy, k, s, (H, W)), be.conv2d_kernel_grad(dy, x, s, pads)
+        assert way == "small" or on_tiled_kernels(tags, shape), tags
+        close(y, exp_f, what="fwd")
+        close(dx, exp_x, what="dx")
         kscale = max(1.0, float(np.abs(exp_k).max()))
-        close(be.conv2d_kernel_grad(dy, x, s, pads), exp_k, scale=kscale, what="dk")
+        close(dk, exp_k, scale=kscale, what="dk")
         if N <= 64:
             exp_f2 = orc.relu_leaky(orc.bias_add(orc.conv2d(x2, k, (s, s)), bias), 0.2)
             got1, got2 = be.conv2d_pair(x, x2, k, (s, s), bias=bias, act=A.ACT_LEAKY, alpha=0.2)
@@ -663,7 +685,9 @@ def test_plans_are_kept_per_geometry(be, orc):
 
     def run(case):
         (N, H, W, C, kh, kw, O, s), x, k, dy, pads, exp = case
-        got = (be.conv2d(x, k, (s, s)), be.conv2d_input_grad(dy, k, s, (H, W)), be.conv2d_kernel_grad(dy, x, s, pads))
+        with convolutions("tiled") as tags:     # (small launches have no plan)
+            got = (be.conv2d(x, k, (s, s)), be.conv2d_input_grad(dy, k, s, (H, W)), be.conv2d_kernel_grad(dy, x, s, pads))
+        assert all(t.startswith("conv_igemm_fast<") for t in tags), tags
         for g, e, what in zip(got, exp, ("fwd", "dx", "dk")):
             close(g, e, scale=max(1.0, float(np.abs(e).max())), what=what)
         return got
@@ -763,8 +787,8 @@ def seeded_geometry(seed):
 
 @pytest.mark.parametrize("seed", range(48))
 def test_seeded_random_geometries(be, orc, seed):
-    """Forward, input gradient and filter gradient of a drawn geometry, with the automatic split and
-    with a drawn forced one, against the oracle."""
+    """Forward, input gradient and filter gradient of a drawn geometry, as the library chooses, on the tiled kernels with their
+    automatic split and with a drawn forced one, against the oracle."""
     import __graft_entry__ as ge
     A = ge.load_package().hipabi
     lib = A.load()
@@ -778,13 +802,15 @@ def test_seeded_random_geometries(be, orc, seed):
     exp_dx = orc.conv2d_input_grad(dy, k, s, (H, W))
     exp_dk = orc.conv2d_kernel_grad(dy, x, s, pads)
     forced = int(np.random.default_rng(seed).integers(2, 7))
-    for splits in (0, forced):
+    for splits, way in ((0, "small"), (0, "tiled"), (forced, "tiled")):
         A.check(lib.dh_debug_force_splitk(splits))
         try:
-            close(be.conv2d(x, k, (s, s)), exp_y, what="fwd, splits %d" % splits)
-            close(be.conv2d_input_grad(dy, k, s, (H, W)), exp_dx, what="dx, splits %d" % splits)
-            close(be.conv2d_kernel_grad(dy, x, s, pads), exp_dk, scale=max(1.0, float(np.abs(exp_dk).max())),
-                  what="dk, splits %d" % splits)
+            with convolutions(way) as tags:
+                y, dx, dk = be.conv2d(x, k, (s, s)), be.conv2d_input_grad(dy, k, s, (H, W)), be.conv2d_kernel_grad(dy, x, s, pads)
+            assert way == "small" or not any(t.startswith("conv_tiny") for t in tags), tags
+            close(y, exp_y, what="fwd, splits %d, %s" % (splits, way))
+            close(dx, exp_dx, what="dx, splits %d, %s" % (splits, way))
+            close(dk, exp_dk, scale=max(1.0, float(np.abs(exp_dk).max())), what="dk, splits %d, %s" % (splits, way))
         finally:
             A.check(lib.dh_debug_force_splitk(0))
 

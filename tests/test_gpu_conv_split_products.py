@@ -6,7 +6,7 @@ gives, in single and paired launches and with either tile width."""
 import numpy as np
 import pytest
 
-from common import RTOL, ATOL, rand_conv_inputs, same_pad
+from common import RTOL, ATOL, convolutions, rand_conv_inputs, same_pad
 
 pytestmark = pytest.mark.gpu
 
@@ -25,6 +25,21 @@ SHAPES = [
     (9, 19, 17, 4, 4, 4, 36, 1),
 ]
 
+# Which kernel forms them: launches as small as these leave the tiled one for conv_tiny, two input gradients are too large for that.
+WAYS = [(shape, way) for shape in SHAPES[:5] for way in ("tiled", "small")] + [(shape, "image") for shape in SHAPES[5:]]
+TOO_LARGE = [(SHAPES[3], "dx"), (SHAPES[4], "dx")]
+IMAGE = dict(zip(SHAPES[5:], [("fwd_rows", "dx_col2im", "dk_thin"), ("fwd_rows", "dx_few_channels", "dk_thin"),
+                              ("fwd_thin", "dx_col2im", "conv_igemm"), ("fwd_thin", "conv_tiny", "dk_thin")]))
+
+
+def kernel_of(way, shape, op):
+    if way == "image":
+        return IMAGE[shape][("fwd", "dx", "dk").index(op)]
+    if way == "small" and (shape, op) not in TOO_LARGE:
+        return "conv_tiny"
+    C, O = shape[3], shape[6]
+    return "conv_igemm_fast" if {"fwd": C % 16 == 0, "dx": O % 16 == 0, "dk": C % 4 == 0 and O % 4 == 0}[op] else "conv_igemm"
+
 
 @pytest.fixture(scope="module")
 def be():
@@ -32,21 +47,41 @@ def be():
     return ge.load_package().HipBackend(0)
 
 
-def products(be, x, k, dy, s):
+def product(be, op, x, k, dy, s):
     H, W = x.shape[1:3]
-    pads = (same_pad(H, k.shape[0], s)[0], same_pad(W, k.shape[1], s)[0])
-    return {"fwd": be.conv2d(x, k, (s, s)), "dx": be.conv2d_input_grad(dy, k, s, (H, W)),
-            "dk": be.conv2d_kernel_grad(dy, x, s, pads)}
+    if op == "fwd":
+        return be.conv2d(x, k, (s, s))
+    if op == "dx":
+        return be.conv2d_input_grad(dy, k, s, (H, W))
+    return be.conv2d_kernel_grad(dy, x, s, (same_pad(H, k.shape[0], s)[0], same_pad(W, k.shape[1], s)[0]))
+
+
+def products(be, x, k, dy, s):
+    return {op: product(be, op, x, k, dy, s) for op in ("fwd", "dx", "dk")}
+
+
+def products_by(be, way, shape, x, k, dy, ops=("fwd", "dx", "dk")):
+    """The products, each by the kernel that `way` names."""
+    import __graft_entry__ as ge
+    if way == "small" and ge.load_package().hipabi.device_info()["compute_units"] != 256:
+        pytest.skip("which launches are small ones is that of a device with 256 compute units")
+    got = {}
+    for op in ops:
+        with convolutions(way) as tags:
+            got[op] = product(be, op, x, k, dy, shape[-1])
+        print("  %s: %s" % (op, tags), flush=True)
+        assert [t.split("<")[0] for t in tags] == [kernel_of(way, shape, op)]
+    return got
 
 
 @pytest.mark.parametrize("scale", ["one", "wide", "tiny"])
-@pytest.mark.parametrize("shape", SHAPES)
-def test_no_less_accurate_than_fp32_products(be, orc64, shape, scale):
+@pytest.mark.parametrize("shape,way", WAYS)
+def test_no_less_accurate_than_fp32_products(be, orc64, shape, way, scale):
     """Error against float64 sums, in the 2-norm over a result of thousands of elements: at most 1.1 times that of
     the fp32 kernel (equal in expectation or better; the ratio of two such norms scatters by a few percent).
     wide: magnitudes over 20 binades, so that the low parts of large values meet the high parts of small ones.
     tiny: activations around 1e-35, whose low parts bf16 holds as subnormals only, unless they are scaled first."""
-    print("shape", shape, scale, flush=True)
+    print("shape", shape, way, scale, flush=True)
     x, k, dy = rand_conv_inputs(11, *shape)
     if scale == "wide":
         rng = np.random.default_rng(12)
@@ -54,7 +89,7 @@ def test_no_less_accurate_than_fp32_products(be, orc64, shape, scale):
     if scale == "tiny":
         x, dy = x * np.float32(1e-35), dy * np.float32(1e-35)
     s = shape[-1]
-    got = products(be, x, k, dy, s)
+    got = products_by(be, way, shape, x, k, dy)
     be.lib.dh_debug_force_generic_conv(1)
     try:
         plain = products(be, x, k, dy, s)
@@ -71,9 +106,9 @@ def test_no_less_accurate_than_fp32_products(be, orc64, shape, scale):
 
 
 @pytest.mark.parametrize("what", ["inf", "nan", "largest"])
-@pytest.mark.parametrize("shape", SHAPES)
-def test_operands_without_finite_parts(be, orc, shape, what):
-    print("shape", shape, what, flush=True)
+@pytest.mark.parametrize("shape,way", WAYS)
+def test_operands_without_finite_parts(be, orc, shape, way, what):
+    print("shape", shape, way, what, flush=True)
     x, k, dy = rand_conv_inputs(13, *shape)
     odd = {"inf": np.inf, "nan": np.nan, "largest": -np.finfo(np.float32).max}[what]
     k[np.abs(k) < 1e-4] = 1e-4    # no infinity times zero that only one order of the sums would meet
@@ -91,7 +126,7 @@ def test_operands_without_finite_parts(be, orc, shape, what):
     s = shape[-1]
     with np.errstate(all="ignore"):
         exp = products(orc, x, k, dy, s)
-    got = products(be, x, k, dy, s)
+    got = products_by(be, way, shape, x, k, dy)
     for op in got:
         g, e = got[op], exp[op]
         np.testing.assert_array_equal(np.isnan(g), np.isnan(e), err_msg=op)
@@ -121,17 +156,17 @@ def products64(x, k, dy, s):
     return {"fwd": y, "dx": dxp[:, pt:pt + H, pl:pl + W], "dk": dk}
 
 
-SPARSE = [(shape, op) for shape in SHAPES for op in ("fwd", "dx", "dk")]
+SPARSE = [(shape, way, op) for shape, way in WAYS for op in ("fwd", "dx", "dk")]
 
 
 @pytest.mark.parametrize("live", ["one", 0.1, 0.5, "positive"])
-@pytest.mark.parametrize("shape,op", SPARSE)
-def test_no_less_accurate_on_sparse_operands(be, shape, op, live):
+@pytest.mark.parametrize("shape,way,op", SPARSE)
+def test_no_less_accurate_on_sparse_operands(be, shape, way, op, live):
     """As above where few of a sum's products are not zero (activations and gradients behind a relu): fp32 rounds
     such a sum once per product, and the parts of one product must not cost more.  one: one product on average;
     positive: all of them, of one sign.  1.1: the three products of parts that are left out add 3 % to the error of a
     single product, the rest is the scatter of two norms over thousands of elements."""
-    print("shape", shape, op, live, flush=True)
+    print("shape", shape, way, op, live, flush=True)
     x, k, dy = rand_conv_inputs(17, *shape)
     s = shape[-1]
     rng = np.random.default_rng(18)
@@ -144,10 +179,10 @@ def test_no_less_accurate_on_sparse_operands(be, shape, op, live):
             dy = np.where(rng.random(dy.shape) < part, dy, np.float32(0))
         else:
             x = np.where(rng.random(x.shape) < part, x, np.float32(0))
-    got = products(be, x, k, dy, s)[op].astype(np.float64)
+    got = products_by(be, way, shape, x, k, dy, (op,))[op].astype(np.float64)
     be.lib.dh_debug_force_generic_conv(1)
     try:
-        plain = products(be, x, k, dy, s)[op].astype(np.float64)
+        plain = product(be, op, x, k, dy, s).astype(np.float64)
     finally:
         be.lib.dh_debug_force_generic_conv(0)
     exact = products64(x, k, dy, s)[op]
@@ -157,12 +192,12 @@ def test_no_less_accurate_on_sparse_operands(be, shape, op, live):
 
 
 @pytest.mark.parametrize("what", ["small times large", "subnormal times large", "small beside ordinary"])
-@pytest.mark.parametrize("shape", SHAPES)
-def test_small_operands(be, shape, what):
+@pytest.mark.parametrize("shape,way", WAYS)
+def test_small_operands(be, shape, way, what):
     """Operands whose parts bf16 holds only in part (below 2^-109) or not at all, where their products count: beside
     a large partner, or as the one small image (filter gradient: the one small channel) of a tile of ordinary ones.
     The slice of the result that they make is as close to float64 sums as the fp32 kernel's (1.1: as above)."""
-    print("shape", shape, what, flush=True)
+    print("shape", shape, way, what, flush=True)
     s = shape[-1]
     x, k, dy = rand_conv_inputs(19, *shape)
     inputs = {"fwd": (x, k, dy), "dx": (x, k, dy), "dk": (x, k, dy)}
@@ -178,10 +213,10 @@ def test_small_operands(be, shape, what):
         small, large = (np.float32(v) for v in ((1e-37, 1e16) if what == "small times large" else (1e-41, 1e20)))
         inputs = {"fwd": (x * small, k * large, dy), "dx": (x, k * large, dy * small), "dk": (x * small, k, dy * large)}
     for op in inputs:
-        got = products(be, *inputs[op], s)[op]
+        got = products_by(be, way, shape, *inputs[op], (op,))[op]
         be.lib.dh_debug_force_generic_conv(1)
         try:
-            plain = products(be, *inputs[op], s)[op]
+            plain = product(be, op, *inputs[op], s)
         finally:
             be.lib.dh_debug_force_generic_conv(0)
         exact = products64(*inputs[op], s)[op][where[op]]
@@ -258,7 +293,7 @@ def test_operands_without_finite_parts_in_paired_launches(be, orc, shape, where,
         np.testing.assert_allclose(g[fine], e[fine], rtol=RTOL, atol=ATOL * max(1.0, float(plain.max(initial=0))), err_msg=op)
 
 
-@pytest.mark.parametrize("pair", [False, True])
+@pytest.mark.parametrize("way", ["tiled", "small", "pair"])
 @pytest.mark.parametrize("shape", [
     (1, 3, 3, 16, 3, 3, 20, 1),       # less than one slab of 16 output pixels
     (5, 1, 1, 48, 1, 1, 8, 1),        # an image a pixel
@@ -267,20 +302,22 @@ def test_operands_without_finite_parts_in_paired_launches(be, orc, shape, where,
     (9, 7, 3, 12, 5, 4, 36, 2),       # a row of two pixels, most taps of a pixel in the padding
     (17, 6, 6, 260, 2, 2, 136, 2),    # 128 x 128 tiles, rows and columns left over
 ])
-def test_filter_gradient_of_any_batch(be, shape, pair):
+def test_filter_gradient_of_any_batch(be, shape, way):
     """Batches that are no multiple of 16: the output pixels of a slab are decoded eight at a time and may belong to any
     rows and images.  Element by element within the error of any fp32 summation of n products (n + 2: their own
     rounding and the last one's)."""
-    print("shape", shape, pair, flush=True)
+    print("shape", shape, way, flush=True)
     H, W, s = shape[1], shape[2], shape[-1]
     (x, k, dy), (x2, _, dy2) = (rand_conv_inputs(seed, *shape) for seed in (37, 41))
     pads = (same_pad(H, shape[4], s)[0], same_pad(W, shape[5], s)[0])
     exact, mag = (products64(f(x), k, f(dy), s)["dk"] for f in (np.asarray, np.abs))
     terms = dy[..., 0].size
-    if pair:
-        got = be.conv2d_kernel_grad_pair(dy, x, dy2, x2, s, pads)
+    if way == "pair":
+        with convolutions(way) as tags:
+            got = be.conv2d_kernel_grad_pair(dy, x, dy2, x2, s, pads)
+        assert tags[0].startswith("conv_igemm_fast<dk"), tags
         exact, mag = (a + products64(f(x2), k, f(dy2), s)["dk"] for a, f in ((exact, np.asarray), (mag, np.abs)))
         terms *= 2
     else:
-        got = be.conv2d_kernel_grad(dy, x, s, pads)
+        got = products_by(be, way, shape, x, k, dy, ("dk",))["dk"]
     assert (np.abs(got - exact) <= (terms + 2) * 2.0 ** -24 * mag).all()

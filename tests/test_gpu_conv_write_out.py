@@ -5,7 +5,7 @@ import numpy as np
 import pytest
 import torch   # before the library: whichever comes first brings the HIP runtime that both use
 
-from common import rand_conv_inputs
+from common import convolutions, rand_conv_inputs
 
 pytestmark = pytest.mark.gpu
 
@@ -124,13 +124,15 @@ def test_many_slices(A, shape, offset):
     (9, 16, 16, 80, 4, 4, 144, 1),   # 18 x 80 slabs and more: shares of 8
 ])
 def test_small_launches(A, shape):
-    """Forward product and input gradient with the library's own split against the same launch cut differently (one slice):
+    """Forward product and input gradient of the tiled kernel with its own split against the same launch cut differently (one slice):
     two orders of the sums differ by at most n 2^-24 of the sum of the magnitudes, here bounded by that of the largest."""
     print("shape", shape, flush=True)
     be = A.HipBackend(0)
     N, H, W, C, kh, kw, O, s = shape
     x, k, dy = rand_conv_inputs(9, *shape)
-    got = be.conv2d(x, k, (s, s)), be.conv2d_input_grad(dy, k, s, (H, W))
+    with convolutions("tiled", level=2) as tags:
+        got = be.conv2d(x, k, (s, s)), be.conv2d_input_grad(dy, k, s, (H, W))
+    assert all(t.startswith(("conv_igemm_fast<", "hbm:")) for t in tags) and any("splitk_reduce" in t for t in tags), tags
     mag = be.conv2d(np.abs(x), np.abs(k), (s, s)), be.conv2d_input_grad(np.abs(dy), np.abs(k), s, (H, W))
     be.lib.dh_debug_force_splitk(1)
     try:
