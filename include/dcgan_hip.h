@@ -64,7 +64,7 @@ int dh_memcpy_h2d(void* dst_device, const void* src_host, size_t bytes);
  * work queued before it, as the blocking copy does.  Copies above 64 MiB wait for `stream` and are then
  * blocking. */
 int dh_memcpy_h2d_staged(void* dst_device, const void* src_host, size_t bytes, void* stream);
-/* Blocking copy to the host, behind what the null stream holds.  From 2 MiB on it goes through 4 MiB of pinned memory per
+/* Blocking copy to the host, behind what the null stream holds.  From 2 MiB on it goes through 8 MiB of pinned memory per
  * device, kept, and up to three threads of its own for the length of the call. */
 int dh_memcpy_d2h(void* dst_host, const void* src_device, size_t bytes);
 int dh_memcpy_d2d(void* dst_device, const void* src_device, size_t bytes, void* stream);
