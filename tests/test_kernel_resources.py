@@ -69,3 +69,11 @@ def test_no_loop_around_a_load(assembly):
             lines = [l.split()[0] for l in body.split("\n") if l.startswith("\t") and l.split()]
             loops = sum(l.startswith("buffer_load") and "s_cbranch_execnz" in lines[i:i + 4] for i, l in enumerate(lines))
             assert loops == 0, (src, name, loops)
+
+
+def test_no_second_copy_of_the_input_gradient(assembly):
+    """The general kernel has a variant for filters of fewer elements than a wide load reads (the last template argument). The input gradient has no such load, and
+    a variant would be a copy of the kernel that nothing launches."""
+    for src, wanted in (("conv_fwd.hip", 4), ("conv_dk.hip", 4), ("conv_dx.hip", 0)):       # one per tile shape
+        names = [name for name, _ in kernels(assembly[src]) if re.search(r"conv_igemmI\w*Li1ELb0EEE", name)]
+        assert len(names) == wanted, (src, names)
