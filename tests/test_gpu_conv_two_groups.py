@@ -1,6 +1,6 @@
 """Launches whose workgroups are two groups of four wavefronts, each with half of the workgroup's k-slabs: shares that are odd or shorter
-than the rest, whole and split, remainders of rows and columns, batches that are and are not a multiple of 16, two operand pairs, an infinity in
-one group's slabs."""
+than the rest, whole and split, remainders of rows and columns, batches that are and are not a multiple of 16, two operand pairs, stride phases of unequal
+length, values that are not finite in one group's slabs."""
 import os
 import shutil
 import subprocess
@@ -8,17 +8,20 @@ import subprocess
 import numpy as np
 import pytest
 
-from common import rand_conv_inputs, same_pad
+from common import convolutions, rand_conv_inputs, same_pad
+from test_gpu_conv_split_products import products64
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 
 # product, instances, (N, H, W, C, kh, kw, O, stride), cut: workgroups' share of slabs and slices of the longest tile
 CASES = [
     ("fwd", 1, (37, 27, 19, 48, 3, 3, 80, 1), (27, 1)),      # whole, 27 slabs: 14 and 13; 37 images, 80 of 128 columns
-    ("fwd", 1, (16, 24, 20, 80, 3, 3, 132, 1), (23, 2)),     # two slices, the second a slab less; 4 columns in the second tile
+    ("fwd", 1, (16, 24, 20, 80, 3, 3, 196, 1), (23, 2)),     # two slices, the second a slab less; 68 columns in the second tile
     ("fwd", 2, (16, 15, 13, 64, 5, 5, 128, 1), (20, 5)),     # pair
-    ("dx", 1, (40, 13, 12, 132, 3, 3, 112, 1), (32, 2)),     # remainder of rows, image-major
+    ("dx", 1, (40, 13, 12, 196, 3, 3, 112, 1), (32, 2)),     # remainder of rows, image-major
     ("dx", 2, (32, 9, 9, 128, 3, 3, 160, 1), (15, 6)),       # pair
+    ("dx", 1, (21, 13, 15, 224, 5, 5, 160, 2), (20, 5)),     # phases of 9, 6, 6 and 4 taps and of different extents
+    ("dx", 2, (32, 13, 11, 100, 5, 5, 144, 2), (18, 5)),     # ... in a pair, a slab is 16 images of one pixel
     ("dk", 1, (6, 33, 31, 20, 5, 5, 68, 1), (8, 48)),        # smallest share, any batch, many slices shared by threads
     ("dk", 1, (16, 19, 17, 20, 5, 5, 68, 1), (8, 41)),       # a slab is 16 images of one pixel
     ("dk", 2, (16, 19, 17, 20, 5, 5, 132, 1), (20, 33)),     # two pairs of operands
@@ -40,6 +43,14 @@ def test_cut_into_two_groups(case, tmp_path_factory):
     out = subprocess.run([exe, what] + [str(v) for v in (N, H, W, C, O, kh, s, instances)], capture_output=True, text=True, check=True).stdout
     groups, per, slices, workgroups = map(int, out.split())
     assert (groups, (per, slices)) == (2, cut) and workgroups <= 256, out
+
+
+def launch(be, what, x, x2, k, dy, dy2, shape, instances):
+    """The product by a launch of 128x128 tiles: what the plans above are plans of."""
+    with convolutions("any") as tags:
+        got = products(be, what, x, x2, k, dy, dy2, shape, instances)
+    assert tags == ["conv_igemm_fast<%s,128x128>" % what]
+    return got
 
 
 def products(be, what, x, x2, k, dy, dy2, shape, instances):
@@ -79,7 +90,7 @@ def test_sums_of_both_groups(be, orc64, case):
     x, k, dy = rand_conv_inputs(51, *shape)
     x2, _, dy2 = rand_conv_inputs(52, *shape)
     orc64.set_threads(8)
-    got = products(be, what, x, x2, k, dy, dy2, shape, instances)
+    got = launch(be, what, x, x2, k, dy, dy2, shape, instances)
     again = products(be, what, x, x2, k, dy, dy2, shape, instances)
     want = exact(orc64, what, x, x2, k, dy, dy2, shape, instances)
     size = exact(orc64, what, *(np.abs(t) for t in (x, x2, k, dy, dy2)), shape, instances)
@@ -104,3 +115,67 @@ def test_infinity_in_one_groups_slabs(be, orc, tap):
     np.testing.assert_array_equal(np.isposinf(got[..., 33]), np.isposinf(want[..., 33]))
     np.testing.assert_array_equal(np.isneginf(got[..., 33]), np.isneginf(want[..., 33]))
     np.testing.assert_allclose(got[..., others], plain[..., others], rtol=0, atol=2.0 ** -23 * 31 * 432 * 0.02)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("odd", [np.inf, np.nan, 1e30])
+@pytest.mark.parametrize("case,instance", [(case, i) for case in CASES for i in range(case[1])])
+def test_values_without_finite_parts(be, orc64, case, instance, odd):
+    """An infinity, a NaN, a value that bf16 parts overflow on, in either instance: one in the first image and one in the last, in the first and in the last channel,
+    where every tap that they meet is inside the image.  Results of a forward product or an input gradient that they reach have them in different slabs; a
+    filter gradient has them at the beginning and at the end of its contraction.  What is not finite is that of plain arithmetic; the rest is as near
+    to 64-bit sums as any fp32 summation of n products, n 2^-24 of the magnitudes (n + 2: their own rounding and the last one's)."""
+    what, instances, shape, _ = case
+    print("case", case, instance, odd, flush=True)
+    N, H, W, C, kh, kw, O, s = shape
+    ins = [list(rand_conv_inputs(seed, *shape)) for seed in (54, 55)]
+    ins[1][1] = ins[0][1]
+    ins[0][1][np.abs(ins[0][1]) < 1e-4] = 1e-4      # no infinity times zero
+    Ho, Wo = ins[0][2].shape[1:3]
+    pt, pl = same_pad(H, kh, s)[0] // 2, same_pad(W, kw, s)[0] // 2
+    if what == "fwd":
+        t = ins[instance][0]
+        t[0, H // 2, W // 2, 0] = odd
+        t[N - 1, H // 2, W // 2, C - 1] = -odd
+    else:                                           # first and last pixel of dy whose window is inside
+        t = ins[instance][2]
+        t[0, -(-pt // s), -(-pl // s), 0] = odd
+        t[N - 1, (H - kh + pt) // s, (W - kw + pl) // s, O - 1] = -odd
+    (x, k, dy), (x2, _, dy2) = ins
+    orc64.set_threads(8)
+    with np.errstate(all="ignore"):
+        want = exact(orc64, what, x, x2, k, dy, dy2, shape, instances)
+        size = exact(orc64, what, *(np.abs(t) for t in (x, x2, k, dy, dy2)), shape, instances)
+    got = launch(be, what, x, x2, k, dy, dy2, shape, instances)
+    terms = {"fwd": kh * kw * C, "dx": kh * kw * O, "dk": N * Ho * Wo * instances}[what]
+    assert odd == 1e30 or not all(np.isfinite(w).all() for w in want)
+    for g, w, m in zip(got, want, size):
+        for kind in (np.isnan, np.isposinf, np.isneginf):
+            np.testing.assert_array_equal(kind(g), kind(w))
+        fine = np.isfinite(w)
+        err, bound = np.abs(g[fine].astype(np.float64) - w[fine]), (terms + 2) * 2.0 ** -24 * m[fine].astype(np.float64)
+        assert (err <= bound).all(), np.max(err / bound)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("case", CASES)
+def test_no_less_accurate_than_fp32_products(be, case):
+    """Error against float64 sums in the 2-norm, at most 1.1 times that of the general kernel, which multiplies in fp32 (the ratio of two such norms
+    scatters by a few percent)."""
+    what, instances, shape, _ = case
+    print("case", case, flush=True)
+    s = shape[-1]
+    (x, k, dy), (x2, _, dy2) = (rand_conv_inputs(seed, *shape) for seed in (56, 57))
+    got = launch(be, what, x, x2, k, dy, dy2, shape, instances)
+    be.lib.dh_debug_force_generic_conv(1)
+    try:
+        plain = [products(be, what, a, None, k, g, None, shape, 1)[0] for a, g in ((x, dy), (x2, dy2))[:instances]]
+    finally:
+        be.lib.dh_debug_force_generic_conv(0)
+    want = [products64(a, k, g, s)[what] for a, g in ((x, dy), (x2, dy2))[:instances]]
+    if what == "dk":
+        plain, want = [sum(plain)], [sum(want)]
+    for g, p, w in zip(got, plain, want):
+        err, yard = np.linalg.norm(g - w), np.linalg.norm(p - w)
+        print("  relative error %.3g, fp32 products %.3g: %.2f" % (err / np.linalg.norm(w), yard / np.linalg.norm(w), err / yard), flush=True)
+        assert err <= 1.1 * yard
