@@ -2,8 +2,10 @@
 and single loads, remainders of rows, columns and of the contraction, fewer steps than wavefronts, stride phases without a tap."""
 import numpy as np
 import pytest
+import torch   # before the library: whichever comes first brings the HIP runtime that both use
 
-from common import rand_conv_inputs, same_pad
+from common import convolutions, rand_conv_inputs, same_pad
+from test_gpu_conv_odd_columns import guarded, result
 from test_gpu_conv_split_products import products64
 
 pytestmark = pytest.mark.gpu
@@ -155,3 +157,65 @@ def test_no_part_of_a_product_is_left_out(A, be, case):
     assert len(tags) == 1 and tags[0].startswith("conv_tiny<" + what)
     exact = products64(x, k, dy, s)[what]
     np.testing.assert_array_less(np.abs(got - exact), 0.5 * np.spacing(np.abs(got)) + 2.0 ** -28 * np.abs(exact) + 1e-300)
+
+
+@pytest.mark.parametrize("apart", ["none", "operand", "filter", "bias", "result", "all"])
+@pytest.mark.parametrize("shape", [
+    (2, 9, 7, 32, 3, 3, 48, 1),     # what the buffer-load kernel would take
+    (2, 9, 7, 24, 3, 3, 40, 1),     # 16-byte loads and stores
+    (1, 11, 10, 36, 3, 3, 44, 2),   # 16-byte stores only
+    (1, 12, 13, 37, 3, 3, 29, 1),   # neither
+])
+@pytest.mark.parametrize("what", ["fwd", "dx", "dk"])
+def test_any_address(A, orc64, what, shape, apart):
+    """Every operand, the bias or the result 4 bytes past a multiple of 16, through every activation, between words that stay as they are.  The product is held to 64-bit
+    sums (bound of test_small_launches), the rest to that product and the bias: exact where the activation is a multiplication or none, else
+    within two roundings of tanh and exp in 32 bits."""
+    print(what, shape, apart, flush=True)
+    N, H, W, C, kh, kw, O, s = shape
+    (ph, Ho), (pw, Wo) = A.same_pad(H, kh, s), A.same_pad(W, kw, s)
+    lib, P = A.load(), torch.Tensor.data_ptr
+    A.check(lib.dh_init(0))
+    x, k, dy = rand_conv_inputs(76, *shape)
+    ncols = C if what == "dx" else O
+    bias = np.random.default_rng(77).standard_normal(ncols).astype(np.float32)
+
+    def placed(a, name):
+        first = int(apart in (name, "all"))
+        whole = torch.full((a.size + 8,), float("nan"), device="cuda")
+        part = whole[first:first + a.size]
+        part.copy_(torch.from_numpy(np.ascontiguousarray(a).reshape(-1)))
+        assert P(part) % 16 == 4 * first
+        return part
+
+    first = int(apart in ("result", "all"))
+    xd, kd, yd, bd = placed(x, "operand"), placed(k, "filter"), placed(dy, "filter" if what == "dk" else "operand"), placed(bias, "bias")
+    shape_out = {"fwd": dy.shape, "dx": x.shape, "dk": k.shape}[what]
+
+    def run(b, act):
+        whole, out = guarded(shape_out, first)
+        if what == "fwd":
+            A.check(lib.dh_conv2d_fwd(P(xd), P(kd), out, N, H, W, C, kh, kw, O, s, s, ph // 2, pw // 2, Ho, Wo, b, act, 0.2, None))
+        elif what == "dx":
+            A.check(lib.dh_conv2d_dx(P(yd), P(kd), out, N, Ho, Wo, O, kh, kw, C, s, s, ph // 2, pw // 2, H, W, b, act, 0.2, None))
+        else:
+            A.check(lib.dh_conv2d_dk(P(xd), P(yd), out, N, H, W, C, Ho, Wo, O, kh, kw, s, s, ph // 2, pw // 2, None))
+        return result(whole, shape_out, first)
+
+    with convolutions("any") as tags:
+        plain = run(None, A.ACT_NONE)
+    assert len(tags) == 1 and tags[0].startswith("conv_tiny<" + what), tags
+    exact, size = (products64(f(x), f(k), f(dy), s)[what] for f in (np.asarray, np.abs))
+    contraction = {"fwd": kh * kw * C, "dx": kh * kw * O, "dk": N * Ho * Wo}[what]
+    assert (np.abs(plain - exact) <= (contraction / 8 / 16 + 12) * 2.0 ** -23 * size).all()
+    if what == "dk":
+        return
+    for b in (None, bias):
+        z = plain if b is None else plain + b
+        for act, want in {A.ACT_NONE: z, A.ACT_RELU: np.where(z < 0, np.float32(0), z), A.ACT_LEAKY: np.where(z < 0, np.float32(0.2) * z, z),
+                          A.ACT_TANH: np.tanh(z.astype(np.float64)), A.ACT_SIGMOID: 1 / (1 + np.exp(-z.astype(np.float64)))}.items():
+            got = run(None if b is None else P(bd), act)
+            if act in (A.ACT_TANH, A.ACT_SIGMOID):
+                np.testing.assert_allclose(got, want, rtol=1e-6, atol=1e-6, err_msg=str(act))
+            else:
+                np.testing.assert_array_equal(got, want, err_msg=str(act))
