@@ -79,7 +79,7 @@ int conv_dx(const char* who, const float* dy, const float* dy2, const float* k, 
     if (!pair)
     {
         const bool fast = takes_fast_path(veca, vecb);
-        const TinyShape tiny = tiny_shape<MODE_DX>(p, all, n_live, fast);
+        const TinyShape tiny = tiny_shape<MODE_DX>(p, all, n_live, fast, veca);
         if (tiny.tm)
         {
             for (int q = 0; q < n_live; ++q)

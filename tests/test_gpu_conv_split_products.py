@@ -29,7 +29,7 @@ SHAPES = [
 WAYS = [(shape, way) for shape in SHAPES[:5] for way in ("tiled", "small")] + [(shape, "image") for shape in SHAPES[5:]]
 TOO_LARGE = [(SHAPES[3], "dx"), (SHAPES[4], "dx")]
 IMAGE = dict(zip(SHAPES[5:], [("fwd_rows", "dx_col2im", "dk_thin"), ("fwd_rows", "dx_few_channels", "dk_thin"),
-                              ("fwd_thin", "dx_col2im", "conv_igemm"), ("fwd_thin", "conv_tiny", "dk_thin")]))
+                              ("fwd_thin", "dx_col2im", "conv_igemm"), ("fwd_thin", "conv_igemm", "dk_thin")]))
 
 
 def kernel_of(way, shape, op):

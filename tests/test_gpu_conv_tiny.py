@@ -12,19 +12,22 @@ pytestmark = pytest.mark.gpu
 
 # product, tile it must take, (N, H, W, C, kh, kw, O, stride)
 CASES = [
-    ("fwd", "16x16,8", (1, 16, 16, 128, 5, 5, 250, 2)),    # 100 steps, 16-byte loads of x, remainder of columns
+    ("fwd", "16x16,8", (1, 16, 16, 128, 5, 5, 252, 2)),    # 100 steps, 16-byte loads of x, remainder of columns
     ("fwd", "16x16,8", (1, 12, 13, 37, 3, 3, 29, 1)),      # 333 k: single loads, a lane's k in two taps
     ("fwd", "32x16,8", (3, 27, 19, 48, 3, 3, 80, 1)),      # 14 steps for 8 wavefronts
     ("fwd", "32x32,8", (20, 33, 33, 18, 4, 4, 30, 2)),
     ("fwd", "32x32,4", (10, 40, 40, 10, 2, 2, 100, 2)),    # 40 k: two steps for four wavefronts
     ("dx", "16x16,8", (1, 32, 32, 64, 5, 5, 128, 2)),      # phases of 9, 6, 6 and 4 taps
     ("dx", "16x16,8", (8, 12, 13, 37, 3, 3, 29, 1)),
-    ("dx", "32x16,8", (2, 32, 32, 64, 5, 5, 128, 2)),
+    ("dx", "32x16,8", (4, 20, 21, 64, 3, 3, 96, 1)),
+    ("dx", "32x16,8", (20, 24, 25, 34, 3, 3, 37, 1)),      # single loads
     ("dx", "32x32,4", (4, 8, 9, 513, 1, 1, 96, 1)),        # one tap
-    ("dx", "32x32,4", (10, 21, 19, 40, 1, 1, 100, 2)),     # three of four phases have no tap: zeros
+    ("dx", "32x32,4", (40, 21, 19, 40, 1, 1, 100, 2)),     # three of four phases have no tap: zeros
+    ("dx", "32x32,8", (6, 24, 25, 64, 3, 3, 64, 1)),
+    ("dx", "32x32,8", (1, 30, 28, 512, 5, 5, 48, 2)),      # fewer steps than wavefronts in some phases
     ("dk", "16x16,8", (1, 12, 13, 37, 3, 3, 29, 1)),
     ("dk", "32x16,8", (4, 16, 16, 64, 5, 5, 64, 2)),
-    ("dk", "32x32,4", (1, 16, 16, 128, 5, 5, 256, 2)),     # two steps for four wavefronts
+    ("dk", "32x32,4", (3, 16, 16, 96, 5, 5, 128, 2)),      # six steps for four wavefronts
     ("dk", "32x32,8", (2, 32, 32, 64, 5, 5, 128, 2)),
 ]
 
@@ -74,6 +77,24 @@ def test_small_launches(A, be, orc64, case):
     contraction = {"fwd": kh * kw * C, "dx": kh * kw * O, "dk": N * H * W}[what]
     bound = (contraction / 8 / 16 + 12) * 2.0 ** -23 * size
     assert (np.abs(got - want) <= bound).all(), np.max(np.abs(got - want) / np.maximum(bound, 1e-300))
+
+
+@pytest.mark.parametrize("case", [   # tiled, us / here, us
+    ("fwd", (44, 25, 25, 92, 3, 3, 16, 1)),     # 27.5 / 42.8: half of a tile's columns past the end
+    ("fwd", (97, 34, 32, 5, 4, 4, 45, 2)),      # 11.8 / 19.6: single loads
+    ("fwd", (7, 29, 29, 192, 5, 5, 48, 2)),     # 23.7 / 29.0
+    ("dx", (420, 8, 6, 48, 1, 1, 112, 1)),      # 9.9 / 11.8: many results, a short contraction
+    ("dk", (141, 7, 7, 113, 5, 5, 43, 2)),      # 27.6 / 34.3
+])
+def test_small_launches_that_tiled_kernels_do_faster(A, be, case):
+    what, shape = case
+    print("case", case, flush=True)
+    if A.device_info()["compute_units"] != 256:
+        pytest.skip("the choice is that of a device with 256 compute units")
+    x, k, dy = rand_conv_inputs(78, *shape)
+    with convolutions("any") as tags:
+        product(be, what, x, k, dy, shape)
+    assert len(tags) == 1 and tags[0].startswith("conv_igemm"), tags
 
 
 @pytest.mark.parametrize("act", ["none", "leaky", "tanh"])
