@@ -1,5 +1,5 @@
-"""Results whose columns are no multiple of 4: the write-out turns 32 x 32 tiles in LDS.  Around the widths where that begins, the tiles' edges and
-remainders, direct and from slices, with and without a result that starts at 16 bytes; nothing outside the result is written."""
+"""Results whose columns are no multiple of 4: the write-out of launches that are large enough turns 32 x 32 tiles in LDS.  Around the widths where that begins, the tiles' edges
+and remainders, direct and from slices, with and without a result that starts at 16 bytes; nothing outside the result is written."""
 import numpy as np
 import pytest
 import torch
@@ -31,6 +31,17 @@ def result(whole, shape, first):
     return got[64 + first:64 + first + n].reshape(shape)
 
 
+def workgroups(rows, columns, slices):
+    bm, bn = (128, 32) if columns <= 32 else (64 if rows <= 64 else 128, 64 if columns <= 64 or rows <= 64 else 128)
+    return -(-rows // bm) * -(-columns // bn) * slices
+
+
+def turned(rows, columns, slices):
+    """The rule of the launch, on a device with 256 units."""
+    return workgroups(rows, columns, slices) * (2 if slices > 1 else 4) >= 256
+
+
+@pytest.mark.parametrize("many", [False, True])      # rows enough that they are turned
 @pytest.mark.parametrize("splits", [1, 3])
 @pytest.mark.parametrize("shape", [      # N, H, W, C, kh, kw, O, stride
     (3, 9, 11, 16, 3, 3, 17, 1),         # the narrowest that is turned
@@ -45,9 +56,13 @@ def result(whole, shape, first):
     (4, 16, 16, 24, 3, 3, 40, 1),        # multiples of 4 at any address
 ])
 @pytest.mark.parametrize("first", [0, 1])
-def test_write_out(A, orc, shape, splits, first):
-    print("shape", shape, "splits", splits, "first", first, flush=True)
+def test_write_out(A, orc, shape, splits, first, many):
     N, H, W, C, kh, kw, O, s = shape
+    if many:
+        N = -(-64 * 128 // (-(-H // s) * -(-W // s)))
+        shape = (N,) + shape[1:]
+    print("shape", shape, "splits", splits, "first", first, flush=True)
+    dk_splits = 160 if many and splits > 1 else splits
     (ph, Ho), (pw, Wo) = A.same_pad(H, kh, s), A.same_pad(W, kw, s)
     x, k, dy = rand_conv_inputs(71, *shape)
     bias, bias_c = np.linspace(-0.5, 0.5, O).astype(np.float32), np.linspace(-0.3, 0.3, C).astype(np.float32)
@@ -61,10 +76,15 @@ def test_write_out(A, orc, shape, splits, first):
     adj = (N, Ho, Wo, O, kh, kw, C, s, s, ph // 2, pw // 2, H, W)
     fil = (N, H, W, C, Ho, Wo, O, kh, kw, s, s, ph // 2, pw // 2)
     (wy, y), (wx, gx), (wk, gk) = (guarded(e.shape, first) for e in exp)
+    if many and A.device_info()["compute_units"] == 256:
+        slices = min(splits, -(-kh * kw * C // 16))
+        assert turned(N * Ho * Wo, O, slices) and (s > 1 or turned(N * H * W, C, min(splits, -(-kh * kw * O // 16))))
+        assert splits == 1 or turned(kh * kw * C, O, dk_splits)
     lib.dh_debug_force_splitk(splits)
     try:
         A.check(lib.dh_conv2d_fwd(p(dx), p(dk), y, *fwd, p(db), A.ACT_LEAKY, 0.2, None))
         A.check(lib.dh_conv2d_dx(p(ddy), p(dk), gx, *adj, p(dbc), A.ACT_TANH, 0.0, None))
+        lib.dh_debug_force_splitk(dk_splits)
         A.check(lib.dh_conv2d_dk(p(dx), p(ddy), gk, *fil, None))
     finally:
         lib.dh_debug_force_splitk(0)
@@ -72,6 +92,25 @@ def test_write_out(A, orc, shape, splits, first):
         # sums of N*Ho*Wo products of U(-1,1) values: the filter gradient's absolute tolerance follows their magnitude
         scale = max(1.0, float(np.abs(e).max())) if what == "dk" else 1.0
         np.testing.assert_allclose(result(whole, e.shape, first), e, rtol=RTOL, atol=ATOL * scale, err_msg=what)
+
+
+@pytest.mark.parametrize("first", [0, 1])
+def test_whole_filter_gradient(A, orc, first):
+    """Turned in one slice: 22 x 3 tiles, both ends a part."""
+    N, H, W, C, kh, kw, O, s = shape = (2, 4, 5, 309, 3, 3, 303, 1)
+    assert turned(kh * kw * C, O, 1)
+    x, k, dy = rand_conv_inputs(73, *shape)
+    orc.set_threads(8)
+    want = orc.conv2d_kernel_grad(dy, x, s, (same_pad(H, kh, s)[0], same_pad(W, kw, s)[0]))
+    xd, yd = (torch.from_numpy(np.ascontiguousarray(a)).cuda() for a in (x, dy))
+    whole, gk = guarded(k.shape, first)
+    lib = A.load()
+    lib.dh_debug_force_splitk(1)
+    try:
+        A.check(lib.dh_conv2d_dk(xd.data_ptr(), yd.data_ptr(), gk, N, H, W, C, H, W, O, kh, kw, s, s, 1, 1, None))
+    finally:
+        lib.dh_debug_force_splitk(0)
+    np.testing.assert_allclose(result(whole, k.shape, first), want, rtol=RTOL, atol=ATOL * max(1.0, float(np.abs(want).max())))
 
 
 @pytest.mark.parametrize("shape", [      # N, H, W, C, kh, kw, O, stride
