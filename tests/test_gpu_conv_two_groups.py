@@ -19,7 +19,7 @@ CASES = [
     ("fwd", 1, (16, 24, 20, 80, 3, 3, 196, 1), (23, 2)),     # two slices, the second a slab less; 68 columns in the second tile
     ("fwd", 2, (16, 15, 13, 64, 5, 5, 128, 1), (20, 5)),     # pair
     ("dx", 1, (40, 13, 12, 196, 3, 3, 112, 1), (32, 2)),     # remainder of rows, image-major
-    ("dx", 2, (32, 9, 9, 128, 3, 3, 160, 1), (15, 6)),       # pair
+    ("dx", 2, (48, 9, 9, 128, 3, 3, 160, 1), (23, 4)),       # pair
     ("dx", 1, (21, 13, 15, 224, 5, 5, 160, 2), (20, 5)),     # phases of 9, 6, 6 and 4 taps and of different extents
     ("dx", 2, (32, 13, 11, 100, 5, 5, 144, 2), (18, 5)),     # ... in a pair, a slab is 16 images of one pixel
     ("dk", 1, (6, 33, 31, 20, 5, 5, 68, 1), (8, 48)),        # smallest share, any batch, many slices shared by threads
@@ -29,9 +29,12 @@ CASES = [
 ]
 
 
-@pytest.mark.parametrize("case", CASES)
-def test_cut_into_two_groups(case, tmp_path_factory):
-    """The launches below are the ones this file is about, and no unit gets two workgroups."""
+# enough slabs for two groups with those in the padding, not without
+NARROW = [("dx", 1, (421, 2, 2, 240, 3, 3, 240, 1)), ("fwd", 2, (160, 3, 2, 208, 5, 5, 96, 1)), ("dx", 2, (208, 2, 4, 128, 4, 4, 176, 1))]
+
+
+def plan(case, tmp_path_factory):
+    """Groups, share, slices and workgroups of a launch of square tiles; 0 groups: it takes narrower ones."""
     hipcc = shutil.which("hipcc") or "/opt/rocm/bin/hipcc"
     if not os.path.exists(hipcc):
         pytest.skip("hipcc not found")
@@ -39,10 +42,21 @@ def test_cut_into_two_groups(case, tmp_path_factory):
     if not os.path.exists(exe):
         subprocess.run([hipcc, "--cuda-host-only", "-O1", "-std=c++17", "-Wno-unused-function", "-I" + os.path.join(ROOT, "include"),
                         "-I" + os.path.join(ROOT, "dcgan-cuda_amd", "csrc"), "-o", exe, os.path.join(ROOT, "tests", "two_groups_plan.hip")], check=True)
-    what, instances, (N, H, W, C, kh, kw, O, s), cut = case
+    what, instances, (N, H, W, C, kh, kw, O, s) = case[:3]
     out = subprocess.run([exe, what] + [str(v) for v in (N, H, W, C, O, kh, s, instances)], capture_output=True, text=True, check=True).stdout
-    groups, per, slices, workgroups = map(int, out.split())
-    assert (groups, (per, slices)) == (2, cut) and workgroups <= 256, out
+    return tuple(map(int, out.split()))
+
+
+@pytest.mark.parametrize("case", CASES)
+def test_cut_into_two_groups(case, tmp_path_factory):
+    """The launches below are the ones this file is about, and no unit gets two workgroups."""
+    groups, per, slices, workgroups = plan(case, tmp_path_factory)
+    assert (groups, (per, slices)) == (2, case[3]) and workgroups <= 256
+
+
+@pytest.mark.parametrize("case", NARROW)
+def test_slabs_in_the_padding_do_not_count(case, tmp_path_factory):
+    assert plan(case, tmp_path_factory)[0] == 0
 
 
 def launch(be, what, x, x2, k, dy, dy2, shape, instances):

@@ -20,7 +20,7 @@ static void show(ConvParams& p, const Phase* phase, int n, bool pair)
             workgroups += slices_of(slab_set<MODE>(p, phase[z], m0, 128, z).count() * k, p.per_split) * copies;
             slabs += (phase[z].K + BK - 1) / BK * copies;
         }
-    const bool square = MODE == MODE_DK || narrower_if_split(TileCfg{128, 128}, p.ncols, tiles, slabs, [&] { return p.groups == 2; }).bn == 128;
+    const bool square = MODE == MODE_DK || narrower_if_split(TileCfg{128, 128}, p.ncols, tiles, slabs, [&] { return planned_in_two_groups<MODE>(p, phase, n, pair, tiles); }).bn == 128;
     printf("%d %d %d %ld\n", square ? p.groups : 0, p.per_split, p.splitk, workgroups);
 }
 
