@@ -32,6 +32,9 @@ CASES = [
 # enough slabs for two groups with those in the padding, not without
 NARROW = [("dx", 1, (421, 2, 2, 240, 3, 3, 240, 1)), ("fwd", 2, (160, 3, 2, 208, 5, 5, 96, 1)), ("dx", 2, (208, 2, 4, 128, 4, 4, 176, 1))]
 
+# as long by the estimate, longer in two groups: 186 / 196, 104 / 111 and 116 / 122 us
+ONE_GROUP = [("dk", 2, (181, 7, 5, 288, 5, 5, 336, 2)), ("dk", 2, (245, 5, 5, 320, 5, 5, 176, 2)), ("dk", 1, (64, 42, 42, 80, 3, 3, 80, 1))]
+
 
 def plan(case, tmp_path_factory):
     """Groups, share, slices and workgroups of a launch of square tiles; 0 groups: it takes narrower ones."""
@@ -57,6 +60,11 @@ def test_cut_into_two_groups(case, tmp_path_factory):
 @pytest.mark.parametrize("case", NARROW)
 def test_slabs_in_the_padding_do_not_count(case, tmp_path_factory):
     assert plan(case, tmp_path_factory)[0] == 0
+
+
+@pytest.mark.parametrize("case", ONE_GROUP)
+def test_filter_gradients_of_long_shares(case, tmp_path_factory):
+    assert plan(case, tmp_path_factory)[0] == 1
 
 
 def launch(be, what, x, x2, k, dy, dy2, shape, instances):
