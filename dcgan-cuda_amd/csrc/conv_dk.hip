@@ -48,7 +48,7 @@ int conv_dk(const char* who, const float* x, const float* dy, const float* x2, c
     if (!pair)
     {
         const bool fast = takes_fast_path(veca, vecb);
-        const TinyShape tiny = tiny_shape<MODE_DK>(p, p.phase, 1, fast, veca);
+        const TinyShape tiny = tiny_shape<MODE_DK>(p, p.phase, 1, fast, veca, as_stream(stream));
         if (tiny.tm)
         {
             g_prof_flops = 2.0 * N * Ho * Wo * O * kh * kw * C;

@@ -79,7 +79,7 @@ int conv_dx(const char* who, const float* dy, const float* dy2, const float* k, 
     if (!pair)
     {
         const bool fast = takes_fast_path(veca, vecb);
-        const TinyShape tiny = tiny_shape<MODE_DX>(p, all, n_live, fast, veca);
+        const TinyShape tiny = tiny_shape<MODE_DX>(p, all, n_live, fast, veca, as_stream(stream));
         if (tiny.tm)
         {
             for (int q = 0; q < n_live; ++q)

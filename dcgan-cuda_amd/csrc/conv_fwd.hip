@@ -43,7 +43,7 @@ int conv_fwd(const char* who, const float* x, const float* x2, const float* k, f
     if (!pair)
     {
         const bool fast = takes_fast_path(veca, vecb);
-        const TinyShape tiny = tiny_shape<MODE_FWD>(p, p.phase, 1, fast, veca);
+        const TinyShape tiny = tiny_shape<MODE_FWD>(p, p.phase, 1, fast, veca, as_stream(stream));
         if (tiny.tm)
         {
             g_prof_flops = 2.0 * N * Ho * Wo * O * kh * kw * C;

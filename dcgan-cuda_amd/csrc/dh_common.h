@@ -22,6 +22,8 @@ constexpr int MAX_ARENAS = 8;
 constexpr int STAGE_SLOTS = 16;                       // pinned staging buffers of dh_memcpy_h2d_staged
 constexpr size_t STAGE_MAX_BYTES = size_t(64) << 20;  // larger copies are plain blocking copies
 int workspace(size_t bytes, void** ptr, hipStream_t stream);
+// Whether workspace() has that much for the stream: it holds it, or may allocate it (an arena of the stream's own or room for one, nothing being captured).
+bool workspace_at_hand(size_t bytes, hipStream_t stream);
 // The current device's fixed scratch buffer (STATIC_SCRATCH_BYTES, part of the code object, never
 // allocated or freed): for entry points that must not allocate.  Every call on a device shares it.
 constexpr size_t STATIC_SCRATCH_BYTES = size_t(2) << 20;

@@ -167,6 +167,31 @@ int workspace(size_t bytes, void** ptr, hipStream_t stream)
     return 0;
 }
 
+bool workspace_at_hand(size_t bytes, hipStream_t stream)
+{
+    if (ensure_init() != 0)
+        return false;
+    {
+        std::lock_guard<std::mutex> lock(g_mu);
+        const DeviceState& st = g_dev[g_cur];
+        bool known = false;
+        for (int i = 0; i < st.n_arenas; ++i)
+            if (st.arena[i].stream == stream)
+            {
+                if (bytes <= st.arena[i].bytes)
+                    return true;
+                known = true;
+            }
+        if (!known && st.n_arenas == MAX_ARENAS)
+            return false;
+    }
+    hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(stream, &capturing) == hipSuccess)
+        return capturing == hipStreamCaptureStatusNone;
+    (void)hipGetLastError();
+    return false;
+}
+
 bool g_force_generic = false;
 bool g_force_tiled = false;
 int g_force_splitk = 0;
